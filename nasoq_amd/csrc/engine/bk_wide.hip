@@ -107,6 +107,13 @@ __device__ inline double w_entry(F l, int j, const T* dd, const T* dsb) {
   return l(j) * dd[j];
 }
 
+// lane `l` (uniform) of a double
+__device__ inline double lane_read(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
 __device__ inline int far_phys(int a, int fstart, const unsigned* mbits, const int* mlog, const int* mphys,
                                int nm) {
   const int b = a - fstart;
@@ -123,18 +130,18 @@ __device__ inline int far_phys(int a, int fstart, const unsigned* mbits, const i
 // 512 threads keep 448 (114,688 rows) with 32-column FP64 or 64-column FP32
 // panels, whose LDS rows are the same 256 bytes.
 template <typename T, int NT, int NBM>
-__global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, int sub, int wcols, const int* super,
-                                                 const int64_t* pi, const int64_t* px, T* valL,
-                                                 T* dval, int* perm_piv, T* Wbase,
-                                                 const int64_t* woff, int* kpos, int* kstart, int* sync,
+__global__ __launch_bounds__(NT) void k_bk_wide(WideSn sn, int G, int nb, int sub, int wcols, T* valL, T* dval,
+                                                 int* perm_piv, T* Wbase, int* kpos, int* kstart, int* sync,
                                                  int* sync_next, uint64_t* ll, uint32_t ebase, int n,
                                                  int* status) {
   constexpr int NW = NT / 64;                   // waves; wave NW - 1 holds the diagonal rows
   constexpr int WCH = NT - 64;                  // far rows per workgroup
   constexpr int WLDA = NBM + 1;                 // padded row length of the diagonal rows
+  constexpr int WLDC = WCH + 16;                // padded column length of the far rows: the k-groups of an MFMA
+                                                // operand read fall into different banks
   constexpr int MBITS_WORDS = 256 * WCH / 32;   // moved-far-row bitmap
   static_assert(NBM <= WNB && NT % 64 == 0 && NT >= 256, "wide panel launch shape");
-  __shared__ T LC[NBM * WCH];       // own far rows, column-major [column][row]
+  __shared__ T LC[NBM * WLDC];       // own far rows, column-major [column][row]
   __shared__ T Ad[NBM * WLDA];      // diagonal rows: L (eliminated) | symmetric A (pending)
   __shared__ T wk[NBM], wi[NBM], td0[NBM], td1[NBM], dd[NBM], dsb[NBM], prow[NBM];
   __shared__ int dphys[NBM];
@@ -151,11 +158,12 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
   // counts from zero, and zeroes the other for the next launch (the launch
   // before used it and has ended; the next has not started)
   if (g == 0 && t == 0) __hip_atomic_store(sync_next, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const int s = list[0];
-  const int c0 = super[s], w = super[s + 1] - c0;
-  const int64_t r = pi[s + 1] - pi[s];
-  T* A = valL + px[s];
-  T* Wp = Wbase + woff[s];
+  // the supernode's shape comes with the launch: the only load before the
+  // panel's own is its first column (and the block's)
+  const int s = sn.s, c0 = sn.c0, w = sn.w;
+  const int64_t r = sn.r;
+  T* A = valL + sn.px;
+  T* Wp = Wbase + sn.woff;
   const T* Pp = Wp + (int64_t)w * wcols;  // this panel's columns with the block's earlier panels applied
   T* scr = Wp + (int64_t)w * wcols + (int64_t)r * nb;
   const int k0 = kpos[s];
@@ -183,37 +191,33 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
   const int fr = fbeg + t;
   int myphys = fr;
 #define AG(i, j) A[(int64_t)(j) * r + (i)]
-#define LCR(j) LC[(j) * WCH + t]
+#define LCR(j) LC[(j) * WLDC + t]
 #define ADR(i, j) Ad[(i) * WLDA + (j)]
 
   // ---- load the panel rows
   // panel column j, row i >= j (with the block's earlier panels applied)
   auto pcol = [&](int i, int j) -> T { return sub ? Pp[(int64_t)j * r + i] : AG(i, k0 + j); };
-  // a thread's loads of a batch issue before its LDS stores (one round trip
-  // per batch rather than per entry)
-  if (hasrow) {
-#pragma unroll
-    for (int j0 = 0; j0 < NBM; j0 += 16) {
-      T v[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) v[q] = (j0 + q < nbe) ? pcol(fr, j0 + q) : (T)0;
-#pragma unroll
-      for (int q = 0; q < 16; ++q)
-        if (j0 + q < nbe) LCR(j0 + q) = v[q];
-    }
-  }
+  // all of a thread's loads issue before its first LDS store: one round trip
   {
-    constexpr int Q = NBM * NBM / NT;
-    T v[Q];
+    // diagonal rows (lower triangle): lane = row, the waves share the columns
+    constexpr int Q = (NBM + NW - 1) / NW;
+    T v[Q], f[NBM];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-      const int idx = t + NT * q, i = idx % nbe, j = idx / nbe;
-      v[q] = idx < nbe * nbe ? ((i >= j) ? pcol(k0 + i, j) : pcol(k0 + j, i)) : (T)0;
+      const int i = ln, j = wv + NW * q;
+      v[q] = (i < nbe && j <= i) ? pcol(k0 + i, j) : (T)0;
     }
 #pragma unroll
+    for (int j = 0; j < NBM; ++j) f[j] = (hasrow && j < nbe) ? pcol(fr, j) : (T)0;
+#pragma unroll
     for (int q = 0; q < Q; ++q) {
-      const int idx = t + NT * q, i = idx % nbe, j = idx / nbe;
-      if (idx < nbe * nbe) ADR(i, j) = v[q];
+      const int i = ln, j = wv + NW * q;
+      if (i < nbe && j <= i) ADR(i, j) = v[q];
+    }
+    if (hasrow) {
+#pragma unroll
+      for (int j = 0; j < NBM; ++j)
+        if (j < nbe) LCR(j) = f[j];
     }
   }
   if (t < NBM) {
@@ -241,7 +245,14 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
   // receive the earlier sub-blocks' contribution as 16x16 FP64 MFMA tiles
   // (far rows: a(i,j) -= sum_c L(i,c) W(j,c); diagonal rows:
   // a(i,j) -= sum_c W(i,c) L(j,c)); inside the sub-block every wave computes
-  // the diagonal rows itself, so the steps need no block barrier.  During
+  // the diagonal rows itself, so the steps need no block barrier.
+  // What bounds the panel is the chain of nbe dependent steps, so a step
+  // keeps its operands in registers.  Per 64-column FP64 panel of the 64^3
+  // KKT (476 panels, workgroup 0, phase stamps): load 8.6 us, MFMA 10.8,
+  // steps 16.4 (0.26 us each), exchange 2.6, pivot search 6.9 (averaged; 6
+  // panels take it), write 9.8.  With the columns in LDS and one sum per
+  // step over the sub-block's earlier columns a launch took 115 us, now 58
+  // (FP32 panels of the 48^3 KKT: 129 -> 59).  During
   // the pass the upper triangle of the diagonal rows holds
   // W(i, j) = L(i, j) d_j (row j, column i) and wk holds 1 / d_j.
   {
@@ -252,68 +263,125 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
       const int ce = min(nbe, cb + OSB);
       if (cb > 0) {
         __syncthreads();
-        const int nft = (fcnt + 15) >> 4;      // far-row tiles (rows < WCH)
-        const int ndt = (nbe - cb + 15) >> 4;  // diagonal-row tiles, rows [cb, 64)
-        for (int tile = wv; tile < nft + ndt; tile += NW) {
-          const bool isfar = tile < nft;
-          const int i0 = isfar ? tile * 16 : cb + (tile - nft) * 16;
-          typename Mfma<T>::acc acc = {0, 0, 0, 0};
-          for (int c = 0; c < cb; c += 4) {
-            const int cc = c + lk;
-            // first operand row = column j of the sub-block, second operand col = row i
-            const T x = isfar ? ADR(cc, cb + li) : ADR(cc, cb + li) * wk[cc];
-            const T y = isfar ? LC[cc * WCH + i0 + li] : ADR(cc, i0 + li);
-            acc = Mfma<T>::mma(x, y, acc);
-          }
-          // acc[e] = C(j = cb + orow(e), i = i0 + li)
-          const int i = i0 + li;
-          for (int e = 0; e < 4; ++e) {
-            const int j = cb + Mfma<T>::orow(e, ln);
-            if (j < ce) {
-              if (isfar) {
-                if (i < fcnt) LC[j * WCH + i] -= acc[e];
-              } else if (i < nbe && i >= j) {
-                ADR(i, j) -= acc[e];
-              }
+        // a wave takes its far-row tiles (rows < WCH) and at most one diagonal
+        // tile (rows [cb, nbe)) in lockstep: independent accumulators hide the
+        // operand loads and the MFMA latency.  Tiles beyond the rows compute
+        // on whatever the LDS holds and store nothing.
+        constexpr int NFT = WCH / 16, TPW = (NFT + NW - 1) / NW;
+        static_assert(WCH % 16 == 0 && NBM / OSB <= NW, "far-row and diagonal tiles per wave");
+        const bool dtile = wv < ((nbe - cb + 15) >> 4);
+        const int id0 = cb + (dtile ? 16 * wv : 0);
+        typename Mfma<T>::acc acc[TPW], accd = {0, 0, 0, 0};
+        int i0[TPW];
+#pragma unroll
+        for (int u = 0; u < TPW; ++u) {
+          acc[u] = typename Mfma<T>::acc{0, 0, 0, 0};
+          i0[u] = 16 * min(wv + NW * u, NFT - 1);
+        }
+        // operands of the next k-step are read while this step's MFMAs run
+        T x, xs, y[TPW], yd;
+        auto fetch = [&](int c) {
+          const int cc = c + lk;
+          // first operand row = column j of the sub-block, second operand col = row i
+          x = ADR(cc, cb + li);
+          xs = x * wk[cc];
+#pragma unroll
+          for (int u = 0; u < TPW; ++u) y[u] = LC[cc * WLDC + i0[u] + li];
+          yd = ADR(cc, id0 + li);
+        };
+        fetch(0);
+        for (int c = 0; c < cb; c += 4) {
+          const T x0 = x, xs0 = xs, yd0 = yd;
+          T y0[TPW];
+#pragma unroll
+          for (int u = 0; u < TPW; ++u) y0[u] = y[u];
+          fetch(c + 4 < cb ? c + 4 : c);
+#pragma unroll
+          for (int u = 0; u < TPW; ++u) acc[u] = Mfma<T>::mma(x0, y0[u], acc[u]);
+          accd = Mfma<T>::mma(xs0, yd0, accd);
+        }
+        // acc[e] = C(j = cb + orow(e), i = i0 + li)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = cb + Mfma<T>::orow(e, ln);
+          if (j < ce) {
+#pragma unroll
+            for (int u = 0; u < TPW; ++u) {
+              const int i = i0[u] + li;
+              if (wv + NW * u < NFT && i < fcnt) LC[j * WLDC + i] -= acc[u][e];
             }
+            const int i = id0 + li;
+            if (dtile && i < nbe && i >= j) ADR(i, j) -= accd[e];
           }
         }
         __syncthreads();
       }
-      for (int kr = cb; kr < ce; ++kr) {
-        double vd = 0.0;
-        if (drow && ln >= kr) {
-          double v = ADR(ln, kr);
-          for (int c = cb; c < kr; ++c) v -= (ADR(c, ln) * wk[c]) * ADR(c, kr);
-          vd = v;
+      // the steps themselves: the sub-block's columns of this lane's far row
+      // (vf) and of diagonal row ln (vd, the same in every wave) in
+      // registers, right-looking; the W row of a step is read across the
+      // lanes (v_readlane), so a step has no LDS access and no barrier on its
+      // critical path: d, its reciprocal, one multiplication, one FMA.
+      // Columns beyond ce run on zeros and are neither tested nor stored.
+      double vf[OSB], vd[OSB], rks = 0.0, ds = 0.0;
+#pragma unroll
+      for (int q = 0; q < OSB; ++q) {
+        const int j = cb + q;
+        vf[q] = (hasrow && j < ce) ? (double)LCR(j) : 0.0;
+        vd[q] = (drow && j < ce && ln >= j) ? (double)ADR(ln, j) : 0.0;
+      }
+      const bool fcand = hasrow && fr < w, dcand = wv == NW - 1 && drow;
+      unsigned fm = 0;  // steps at which one of this lane's rows breaks the test
+      double d = lane_read(vd[0], cb), rk = 1.0 / d;
+#pragma unroll
+      for (int q = 0; q < OSB; ++q) {
+        const int kr = cb + q;
+        // W and L entries as they are stored (in T)
+        const T wT = (T)vd[q];
+        const double wd = (double)wT, lf = (double)(T)(vf[q] * rk), ld = (double)(T)(wT * (T)rk);
+        // the next step's pivot first: its reciprocal runs beside the other
+        // columns' updates
+        double dn = 0.0, rkn = 0.0;
+        if (q + 1 < OSB) {
+          const double wj = lane_read(wd, kr + 1);
+          vf[q + 1] -= lf * wj;
+          vd[q + 1] -= ld * wj;
+          dn = lane_read(vd[q + 1], kr + 1);
+          rkn = 1.0 / dn;
         }
-        double v0 = 0.0;
-        if (hasrow) {
-          double v = LCR(kr);
-          for (int c = cb; c < kr; ++c) v -= LCR(c) * ADR(c, kr);
-          v0 = v;
+#pragma unroll
+        for (int j = q + 2; j < OSB; ++j) {
+          const double wj = lane_read(wd, cb + j);
+          vf[j] -= lf * wj;
+          vd[j] -= ld * wj;
         }
-        const double d = __shfl(vd, kr, 64);
         const double absakk = fabs(d);
-        if (!(absakk > 0.0)) myfail = min(myfail, kr);
-        if (wv == NW - 1 && drow && ln > kr) {
-          const double x = fabs(vd);
-          if (x == x && !(absakk >= BK_ALPHA * x)) myfail = min(myfail, kr);
+        const bool bad = !(absakk > 0.0) | (fcand & (BK_ALPHA * fabs(vf[q]) > absakk)) |
+                         (dcand & (ln > kr) & (BK_ALPHA * fabs(vd[q]) > absakk));
+        fm |= bad ? 1u << q : 0u;
+        // keep the updates at this step: sunk to the column's own step they
+        // would need every step's W row in scalar registers
+#pragma unroll
+        for (int j = q + 1; j < OSB; ++j) __asm__ volatile("" : "+v"(vf[j]), "+v"(vd[j]));
+        vf[q] = lf;
+        vd[q] = wd;
+        rks = ln == q ? rk : rks;
+        ds = ln == q ? d : ds;
+        d = dn;
+        rk = rkn;
+      }
+      fm &= (1u << (ce - cb)) - 1u;
+      if (fm) myfail = min(myfail, cb + __ffs(fm) - 1);
+#pragma unroll
+      for (int q = 0; q < OSB; ++q) {
+        const int kr = cb + q;
+        if (kr < ce) {
+          if (hasrow) LCR(kr) = (T)vf[q];
+          if (wv == NW - 1 && drow && ln > kr) ADR(kr, ln) = (T)vd[q];
         }
-        if (hasrow && fr < w) {
-          const double x = fabs(v0);
-          if (x == x && !(absakk >= BK_ALPHA * x)) myfail = min(myfail, kr);
-        }
-        const double rk = 1.0 / d;
-        if (hasrow) LCR(kr) = v0 * rk;
-        if (drow && ln > kr) ADR(kr, ln) = vd;  // every wave stores the same value
-        if (ln == 0) {
-          wk[kr] = rk;
-          dd[kr] = d;
-        }
-        // LDS accesses of one wave complete in order; keep the compiler from
-        // moving the next step's loads above these stores
-        __asm__ volatile("" ::: "memory");
+      }
+      if (wv == NW - 1 && ln < ce - cb) {
+        wk[cb + ln] = (T)rks;
+        dd[cb + ln] = (T)ds;
       }
     }
     if (myfail < nbe) atomicMin(&s_fail, myfail);
@@ -338,13 +406,15 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
   const int J = bci[2];
   // back to the pivoting loop's layout: L below the diagonal for the
   // accepted columns, the original columns from J on
-  if (J < nbe && hasrow)
-    for (int j = J; j < nbe; ++j) LCR(j) = pcol(fr, j);
-  for (int idx = t; idx < nbe * nbe; idx += NT) {
-    const int i = idx % nbe, j = idx / nbe;
-    if (min(i, j) >= J) ADR(i, j) = i >= j ? pcol(k0 + i, j) : pcol(k0 + j, i);
-    else if (i > j) ADR(i, j) = ADR(j, i) * wk[j];
-    else if (i == j) ADR(i, i) = 1.0;
+  if (J < nbe) {
+    if (hasrow)
+      for (int j = J; j < nbe; ++j) LCR(j) = pcol(fr, j);
+    for (int idx = t; idx < nbe * nbe; idx += NT) {
+      const int i = idx % nbe, j = idx / nbe;
+      if (min(i, j) >= J) ADR(i, j) = i >= j ? pcol(k0 + i, j) : pcol(k0 + j, i);
+      else if (i > j) ADR(i, j) = ADR(j, i) * wk[j];
+      else if (i == j) ADR(i, i) = 1.0;
+    }
   }
   if (g == 0 && t < J) {
     dval[c0 + k0 + t] = dd[t];
@@ -408,7 +478,7 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
       }
       if (cand && ai >= fbeg && ai < fbeg + fcnt && absakk < BK_ALPHA * av && t < nbe) {
         uint64_t* pay = ll + LL_PAY + ((int64_t)par * 256 + g) * 2 * WNB;
-        ll_store_d(pay + 2 * t, LC[t * WCH + (ai - fbeg)], fA);
+        ll_store_d(pay + 2 * t, LC[t * WLDC + (ai - fbeg)], fA);
       }
     }
     if (wv == 0) {
@@ -665,7 +735,9 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
   if (t == 0 && s_abort) atomicOr(status, 4);
 
   // ---- moved indices of this panel: (logical, physical)
-  if (t == 0) {
+  const bool plain = J == nbe;  // every step a 1x1 pivot in place: nothing moved
+  if (t == 0 && plain) s_nM = s_nMa = 0;
+  if (t == 0 && !plain) {
     int c = 0, ca = 0;
     for (int i = 0; i < nbe; ++i)
       if (dphys[i] != k0 + i && k0 + i >= kend) {
@@ -743,13 +815,31 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
   }
   // ---- L of the panel and W = L D for the rows of the trailing block
   if (hasrow) {
-    for (int j = 0; j < ker; ++j) {
-      AG(fr, k0 + j) = LCR(j);
-      if (fr < w) Wp[(int64_t)(off + j) * w + fr] = w_entry([&](int c) { return LCR(c); }, j, dd, dsb);
+    if (plain) {  // all pivots 1x1: W is a scaling, sixteen columns' stores together
+      for (int j0 = 0; j0 < ker; j0 += 16) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          const int j = j0 + q;
+          if (j < ker) {
+            const T l = LCR(j);
+            AG(fr, k0 + j) = l;
+            if (fr < w) Wp[(int64_t)(off + j) * w + fr] = l * dd[j];
+          }
+        }
+      }
+    } else {
+      for (int j = 0; j < ker; ++j) {
+        AG(fr, k0 + j) = LCR(j);
+        if (fr < w) Wp[(int64_t)(off + j) * w + fr] = w_entry([&](int c) { return LCR(c); }, j, dd, dsb);
+      }
     }
   }
   for (int idx = gt; idx < nbe * ker; idx += GT) {
     const int i = idx % nbe, j = idx / nbe;
+    if (plain) {  // the upper triangle still holds W(i, j) at (j, i); ker == nbe: no W row is read again
+      if (j <= i) AG(k0 + i, k0 + j) = i > j ? (T)(ADR(j, i) * wk[j]) : (T)1;
+      continue;
+    }
     if (j <= i) AG(k0 + i, k0 + j) = ADR(i, j);
     if (k0 + i >= kend) Wp[(int64_t)(off + j) * w + k0 + i] = w_entry([&](int c) { return ADR(i, c); }, j, dd, dsb);
   }
@@ -763,15 +853,13 @@ __global__ __launch_bounds__(NT) void k_bk_wide(const int* list, int G, int nb, 
 }
 
 template <typename T>
-void launch_bk_wide(const int* list, int G, int nt, int nb, int sub, int wcols, const SnArgs& a, T* valL, T* dval,
-                    int* perm_piv, T* W, const int64_t* woff, int* kpos, int* kstart, int* sync,
-                    int* sync_next, uint64_t* ll, uint32_t ebase, int* status, hipStream_t st) {
+void launch_bk_wide(const WideSn& sn, int G, int nt, int nb, int sub, int wcols, int n, T* valL, T* dval,
+                    int* perm_piv, T* W, int* kpos, int* kstart, int* sync, int* sync_next, uint64_t* ll,
+                    uint32_t ebase, int* status, hipStream_t st) {
   if (nb > wide_panel_nb(nt, sizeof(T)) || nb < 4 || G < 1 || G > 256 || (nt != 256 && nt != WIDE_NT_TALL))
     throw std::runtime_error("bk_wide: launch shape out of range");
-  int n = a.n;
-  void* args[] = {(void*)&list, (void*)&G, (void*)&nb, (void*)&sub, (void*)&wcols, (void*)&a.super, (void*)&a.pi, (void*)&a.px,
-                  (void*)&valL, (void*)&dval, (void*)&perm_piv, (void*)&W, (void*)&woff,
-                  (void*)&kpos, (void*)&kstart, (void*)&sync, (void*)&sync_next, (void*)&ll, (void*)&ebase, (void*)&n,
+  void* args[] = {(void*)&sn, (void*)&G, (void*)&nb, (void*)&sub, (void*)&wcols, (void*)&valL, (void*)&dval,
+                  (void*)&perm_piv, (void*)&W, (void*)&kpos, (void*)&kstart, (void*)&sync, (void*)&sync_next, (void*)&ll, (void*)&ebase, (void*)&n,
                   (void*)&status};
   // tall supernodes: 448 far rows per workgroup in the same 256-byte LDS rows
   // (32 FP64 or 64 FP32 columns)
@@ -780,11 +868,9 @@ void launch_bk_wide(const int* list, int G, int nt, int nb, int sub, int wcols, 
   hipError_t e = hipLaunchCooperativeKernel(fn, dim3(G), dim3(nt), args, 0, st);
   if (e != hipSuccess) throw std::runtime_error(std::string("bk_wide: ") + hipGetErrorString(e));
 }
-template void launch_bk_wide<double>(const int*, int, int, int, int, int, const SnArgs&, double*, double*, int*,
-                                     double*, const int64_t*, int*, int*, int*, int*, uint64_t*, uint32_t, int*,
-                                     hipStream_t);
-template void launch_bk_wide<float>(const int*, int, int, int, int, int, const SnArgs&, float*, float*, int*,
-                                    float*, const int64_t*, int*, int*, int*, int*, uint64_t*, uint32_t, int*,
-                                    hipStream_t);
+template void launch_bk_wide<double>(const WideSn&, int, int, int, int, int, int, double*, double*, int*, double*,
+                                     int*, int*, int*, int*, uint64_t*, uint32_t, int*, hipStream_t);
+template void launch_bk_wide<float>(const WideSn&, int, int, int, int, int, int, float*, float*, int*, float*,
+                                    int*, int*, int*, int*, uint64_t*, uint32_t, int*, hipStream_t);
 
 }  // namespace lblg

@@ -53,6 +53,7 @@ struct FactorLevel {
   int* d_large = nullptr;
   std::vector<int> large_G, large_nb;  // workgroups and panel width per large supernode
   std::vector<int> large_nt, large_wsub;  // workgroup size and panels per trailing update
+  std::vector<int64_t> large_woff;        // workspace offset
   // host copies of the lists (the path-restricted refactorization filters them)
   std::vector<int> h_small, h_off, h_sch, h_schb;
   std::vector<int64_t> h_schb_ldoff;  // offset of each schur_big supernode's L D block

@@ -433,6 +433,7 @@ static void setup(Handle& h) {
           F.large_nb.push_back(nb);
           F.large_nt.push_back(nt);
           F.large_wsub.push_back(wsub);
+          F.large_woff.push_back(woff[s]);
         }
       }
       if (r > w) {
@@ -858,6 +859,7 @@ static void factor_level(Handle& h, FactorLevel& F, const LevelLists& L, const S
     const int rounds = (w + nb - 2) / (nb - 1) + 1;
     const int wsub = F.large_wsub[q];
     const int wcols = wsub * nb;
+    const WideSn wsn{s, S.super[s], w, r, S.p[S.super[s]], F.large_woff[q]};
     for (int p = 0; p < rounds; ++p) {
       // panels run in blocks of wsub: before panel p of a block, its columns
       // receive the block's earlier panels; the rest of the trailing block is
@@ -887,8 +889,8 @@ static void factor_level(Handle& h, FactorLevel& F, const LevelLists& L, const S
       const uint32_t eb = D.ll_epoch;
       D.ll_epoch += 3u * (uint32_t)nb + 8u;
       timed(D, "bk_panel_group", [&] {
-        launch_bk_wide(F.d_large + q, Gp, nt, nb, sub, wcols, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos,
-                       D.kstart, D.sync + D.wide_par, D.sync + (D.wide_par ^ 1), D.ll, eb, D.status, st);
+        launch_bk_wide(wsn, Gp, nt, nb, sub, wcols, a.n, valL, dval, D.perm_piv, Wb, D.kpos, D.kstart,
+                       D.sync + D.wide_par, D.sync + (D.wide_par ^ 1), D.ll, eb, D.status, st);
       });
       D.wide_par ^= 1;
       if (sub == wsub - 1 || p == rounds - 1) {

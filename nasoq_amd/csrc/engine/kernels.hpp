@@ -71,10 +71,14 @@ constexpr int WIDE_MOVED = 128;     // moved indices per panel (scratch rows)
 // columns of a 256-byte LDS row (32 FP64, 64 FP32)
 inline int wide_panel_nb(int nt, size_t value_size) { return nt == 256 ? 64 : (value_size == 8 ? 32 : 64); }
 constexpr int64_t LL_WORDS = 2 * 256 * 4 + 2 * 256 * 8 + 2 * 256 * 2 * 64;
+struct WideSn {  // one wide supernode: first column, width, rows, offsets of its panel and workspace
+  int s, c0, w;
+  int64_t r, px, woff;
+};
 template <typename T>
-void launch_bk_wide(const int* list, int G, int nt, int nb, int sub, int wcols, const SnArgs& a, T* valL, T* dval,
-                    int* perm_piv, T* W, const int64_t* woff, int* kpos, int* kstart, int* sync,
-                    int* sync_next, uint64_t* ll, uint32_t ebase, int* status, hipStream_t st);
+void launch_bk_wide(const WideSn& sn, int G, int nt, int nb, int sub, int wcols, int n, T* valL, T* dval,
+                    int* perm_piv, T* W, int* kpos, int* kstart, int* sync, int* sync_next, uint64_t* ll,
+                    uint32_t ebase, int* status, hipStream_t st);
 template <typename T>
 void launch_trailing(const int* list, int count, int tiles_per_sn, int lo, const SnArgs& a, T* valL,
                      const T* W, const int64_t* woff, const int* kpos, const int* kstart,

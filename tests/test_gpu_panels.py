@@ -1,0 +1,69 @@
+"""Panel factorizations of supernodes wider than 64 columns against the
+oracle, at the edges of their tiles: widths around the panel, sub-block and
+workgroup sizes, with rows below the diagonal block, every step a 1x1 pivot
+in place or one column whose zero diagonal forces a pivot search there."""
+import numpy as np
+import pytest
+
+from nasoq_amd import lbl
+from nasoq_amd import problems as P
+
+from test_gpu_lbl import check_factor
+
+pytestmark = pytest.mark.gpu
+
+
+def bordered(w, m2, zero_at):
+    """Two dense w-column blocks with m2 common rows below: supernodes w wide
+    with w + m2 rows, and w + m2 wide; zero_at: columns of each block whose
+    diagonal is 0."""
+    n, Ap, Ai, Ax, B = P.tall_border(2 * w, m2, chains=2, seed=w, nrhs=1)
+    Ax = Ax.copy()
+    for z in zero_at:
+        for c in (z, w + z):
+            Ax[Ap[c]] = 0.0
+    return n, Ap, Ai, Ax, B
+
+
+def run(oracle, w, m2, zero_at, precision=lbl.F64):
+    n, Ap, Ai, Ax, B = bordered(w, m2, zero_at)
+    print(f"case panel w={w} m2={m2} zero_at={zero_at} precision={precision}", flush=True)
+    s = lbl.SolverSettings(n, Ap, Ai, Ax)
+    s.reg_diag, s.regularization, s.precision = 1e-9, 0, precision
+    s.n_relax, s.z_relax = [0, 0, 0], [0.0, 0.0, 0.0]  # the blocks' supernodes stay apart
+    assert s.symbolic_analysis(perm=np.arange(n, dtype=np.int32)) == 1
+    assert s.numerical_factorization() == 1
+    assert s.sym_scalar("max_sup_wid") == w + m2  # the second block and the border are one supernode
+    return s, n, Ap, Ai, Ax, B
+
+
+WIDTHS = [65, 79, 80, 81, 96, 127, 129, 192, 255, 257, 321]
+
+
+@pytest.mark.parametrize("group_w", [64, 4096])  # 64: cooperative panels; 4096: one workgroup per supernode
+@pytest.mark.parametrize("w", WIDTHS)
+def test_panel_widths(oracle, w, group_w, monkeypatch):
+    monkeypatch.setenv("LBLG_GROUP_W", str(group_w))
+    for zero_at in ((), (0,), (17,), (w - 1,), (31, 32, w // 2)):
+        s, n, Ap, Ai, Ax, B = run(oracle, w, 37, zero_at)
+        # reg_diag off: the zero diagonals reach the pivot search as they are
+        check_factor(oracle, s, n, Ap, Ai, Ax, 0.0)
+        x = s.solve_only(B[:, 0])
+        assert oracle.backward_error(n, Ap, Ai, Ax, x, B[:, 0]) <= 1e-12
+        s.close()
+
+
+@pytest.mark.parametrize("group_w", [64, 4096])
+def test_panel_float(oracle, group_w, monkeypatch):
+    # the FP32 factor on the same shapes, refined to an FP64 backward error
+    monkeypatch.setenv("LBLG_GROUP_W", str(group_w))
+    for w in (65, 130, 300):
+        n, Ap, Ai, Ax, B = bordered(w, 37, (17,))
+        print(f"case float panel w={w} group_w={group_w}", flush=True)
+        s = lbl.SolverSettings(n, Ap, Ai, Ax)
+        s.reg_diag, s.precision, s.target_bwd_err = 1e-9, lbl.F32, 1e-12
+        assert s.symbolic_analysis(perm=np.arange(n, dtype=np.int32)) == 1
+        assert s.numerical_factorization() == 1
+        x = s.solve_only(B[:, 0])
+        assert oracle.backward_error(n, Ap, Ai, Ax, x, B[:, 0]) <= 1e-12
+        s.close()
