@@ -404,7 +404,7 @@ static void setup(Handle& h) {
         if (w <= group_w) {
           F.medium.push_back(s);
           D.s_kind[s] = 1;
-          wsum += (int64_t)w * PANEL_NB + 2 * (int64_t)w + 16;
+          wsum += (int64_t)w * ONE_WCOLS + ONE_WCOLS * ONE_WCOLS + 16;
         } else {
           // cooperative panel over G workgroups, <= WIDE_ROWS far rows each
           // (the diagonal block below the panel and the off-diagonal rows);
@@ -708,7 +708,6 @@ static void setup(Handle& h) {
     D.ss_max_nnz = h.tune.small_nnz;
     D.graphs = env_int("LBLG_GRAPH", 1) != 0;
     D.schur_direct = env_int("LBLG_SCHUR_DIRECT", 1) != 0;
-    D.panel_lds = env_int("LBLG_PANEL_LDS", 1) != 0;
     D.path_refactor = env_int("LBLG_PATH_REFACTOR", 1) != 0;
     D.trailing_direct = env_int("LBLG_TRAILING_DIRECT", 1) != 0;
     D.strip64 = env_int("LBLG_STRIP_TILE64", 1) != 0;
@@ -832,21 +831,27 @@ static void factor_level(Handle& h, FactorLevel& F, const LevelLists& L, const S
   timed(D, "bk_small", [&] { launch_bk_small(L.small, L.nsmall, L.small_wmax, a, valL, dval, D.perm_piv, D.status, st); });
   // medium supernodes: one workgroup each, panel by panel
   if (L.nmedium > 0) {
+    // each panel eliminates at least nb - 1 columns (a 2x2 pivot never
+    // straddles panels), so panel p starts at column >= lo; the last one
+    // (at most nb rows left) ends its supernode
     const int wmax = L.medium_wmax;
-    const int rounds = (wmax + PANEL_NB - 2) / (PANEL_NB - 1) + 1;
-    // diagonal blocks of at most panel_lds_rows rows: the panel in LDS
-    const int lds_rows = (D.panel_lds && wmax <= panel_lds_rows<T>()) ? wmax : 0;
-    for (int p = 0; p < rounds; ++p) {
+    for (int lo = 0;;) {
+      const int left = wmax - lo;
+      const int one = one_panel_nb<T>(left), nb = one ? one : PANEL_NB;
       timed(D, "bk_panel", [&] {
-        launch_bk_panel(L.medium, L.nmedium, 1, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart, D.sync,
-                        D.status, false, lds_rows, st);
+        if (one)
+          launch_bk_one(L.medium, L.nmedium, left, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart,
+                        D.status, st);
+        else
+          launch_bk_panel(L.medium, L.nmedium, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart, D.sync,
+                          D.status, st);
       });
-      const int lo = std::min(wmax, (p + 1) * (PANEL_NB - 1));
+      if (left <= nb) break;
+      lo += nb - 1;
       const int nt = (wmax - lo + 63) / 64;
-      if (nt > 0)
-        timed(D, "trailing", [&] {
-          launch_trailing(L.medium, L.nmedium, nt * (nt + 1) / 2, lo, a, valL, Wb, D.woff, D.kpos, D.kstart, st);
-        });
+      timed(D, "trailing", [&] {
+        launch_trailing(L.medium, L.nmedium, nt * (nt + 1) / 2, lo, a, valL, Wb, D.woff, D.kpos, D.kstart, st);
+      });
     }
   }
   // large supernodes: a cooperative group of workgroups each, one at a time
@@ -887,7 +892,7 @@ static void factor_level(Handle& h, FactorLevel& F, const LevelLists& L, const S
       const int far = (int)(r - std::min<int64_t>(w, (int64_t)p * (nb - 1) + nb));
       const int Gp = std::min(G, std::max(1, (far + rows - 1) / rows));
       const uint32_t eb = D.ll_epoch;
-      D.ll_epoch += 3u * (uint32_t)nb + 8u;
+      D.ll_epoch += 4u * (uint32_t)nb + 8u;  // 3 per step, one per optimistic pass
       timed(D, "bk_panel_group", [&] {
         launch_bk_wide(wsn, Gp, nt, nb, sub, wcols, a.n, valL, dval, D.perm_piv, Wb, D.kpos, D.kstart,
                        D.sync + D.wide_par, D.sync + (D.wide_par ^ 1), D.ll, eb, D.status, st);

@@ -380,25 +380,19 @@ void launch_bk_small(const int* list, int count, int wmax, const SnArgs& a, T* v
 // Per-supernode workspace at W + woff[s]:  Wp (w x NB, ld w) | t0 (w) | t1 (w)
 //                                         | part (2 G doubles) | parti (2 G ints)
 //
-// LDSP (one workgroup per supernode, diagonal block of at most ldsm rows):
-// the panel's columns [k0, k0 + NB) of the diagonal block's rows [k0, w),
-// its W columns and t0 / t1 live in LDS for the whole panel, so each column
-// step reads and writes LDS only; the panel and W (rows the trailing update
-// reads) are written back at the end.  Entries outside the staged block
-// (earlier panels, later columns, the rows below the diagonal block) stay
-// in memory.
+// This form, with the panel in memory, takes the diagonal blocks with more
+// rows left than a one-workgroup panel's LDS holds (bk_wide.hip, ONE).
 // --------------------------------------------------------------------------
 constexpr int PANEL_UF = 8;  // left-looking terms whose loads are issued together
 
-template <typename T, bool LDSP>
+template <typename T>
 __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const int* super,
                                                   const int64_t* pi, const int64_t* px, T* valL,
                                                   T* dval, int* perm_piv, T* Wbase,
                                                   const int64_t* woff, int* kpos, int* kstart,
-                                                  int* sync, int n, int* status, int ldsm) {
+                                                  int* sync, int n, int* status) {
   __shared__ double sv[8];
   __shared__ int si[8];
-  extern __shared__ double panel_smem[];
   const int sidx = blockIdx.x / G, g = blockIdx.x % G;
   const int s = list[sidx];
   const int c0 = super[s], w = super[s + 1] - c0;
@@ -412,60 +406,24 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
   const int k0 = kpos[s];
   if (k0 >= w) return;  // whole group returns together (k0 is uniform)
   const bool last = (w - k0) <= PANEL_NB;
-  const int pc1 = min(w, k0 + PANEL_NB);  // end of the panel's columns
-  // LDS blocks (LDSP): As(i, j) = L(k0 + i, k0 + j), Ws likewise, ld ldsm
-  T* As = reinterpret_cast<T*>(panel_smem);
-  T* Ws = As + (int64_t)PANEL_NB * ldsm;
-  T* t0 = LDSP ? Ws + (int64_t)PANEL_NB * ldsm - k0 : Wp + (int64_t)w * PANEL_NB;  // indexed by row i >= k0
-  T* t1 = LDSP ? Ws + (int64_t)PANEL_NB * ldsm + ldsm - k0 : Wp + (int64_t)w * PANEL_NB + w;
-  // element (i, j) of the diagonal block / rows below, wherever it lives
-  auto AA = [&](int64_t i, int64_t j) -> T& {
-    if (LDSP && j >= k0 && j < pc1 && i >= k0 && i < w) return As[(j - k0) * ldsm + (i - k0)];
-    return A[j * r + i];
-  };
-  auto WW = [&](int64_t i, int64_t j) -> T& {
-    if (LDSP) return Ws[(j - k0) * ldsm + (i - k0)];
-    return Wp[(j - k0) * w + i];
-  };
-  if (LDSP) {
-    for (int64_t e = threadIdx.x; e < (int64_t)(pc1 - k0) * (w - k0); e += 256) {
-      const int64_t j = e / (w - k0), i = e % (w - k0);
-      As[j * ldsm + i] = A[(k0 + j) * r + (k0 + i)];
-    }
-    __syncthreads();
-  }
+  T* t0 = Wp + (int64_t)w * PANEL_NB;  // indexed by row i >= k0
+  T* t1 = Wp + (int64_t)w * PANEL_NB + w;
+  auto AA = [&](int64_t i, int64_t j) -> T& { return A[j * r + i]; };
+  auto WW = [&](int64_t i, int64_t j) -> T& { return Wp[(j - k0) * w + i]; };
   // v - sum_{j in [k0, k)} L(i, j) W(q, j) for a row i >= k and a row q of W
   auto left_update = [&](T v, int i, int q, int k) -> T {
-    if (LDSP) {
-      const T* ar = As + (i - k0);
-      const T* wr = Ws + (q - k0);
-      const int nk = k - k0;
-      int j = 0;
-      for (; j + PANEL_UF <= nk; j += PANEL_UF) {
-        T av[PANEL_UF], wv[PANEL_UF];
+    int j = k0;
+    for (; j + PANEL_UF <= k; j += PANEL_UF) {
+      T av[PANEL_UF], wv[PANEL_UF];
 #pragma unroll
-        for (int u = 0; u < PANEL_UF; ++u) {
-          av[u] = ar[(int64_t)(j + u) * ldsm];
-          wv[u] = wr[(int64_t)(j + u) * ldsm];
-        }
-#pragma unroll
-        for (int u = 0; u < PANEL_UF; ++u) v -= av[u] * wv[u];
+      for (int u = 0; u < PANEL_UF; ++u) {
+        av[u] = A[(int64_t)(j + u) * r + i];
+        wv[u] = Wp[(int64_t)(j + u - k0) * w + q];
       }
-      for (; j < nk; ++j) v -= ar[(int64_t)j * ldsm] * wr[(int64_t)j * ldsm];
-    } else {
-      int j = k0;
-      for (; j + PANEL_UF <= k; j += PANEL_UF) {
-        T av[PANEL_UF], wv[PANEL_UF];
 #pragma unroll
-        for (int u = 0; u < PANEL_UF; ++u) {
-          av[u] = A[(int64_t)(j + u) * r + i];
-          wv[u] = Wp[(int64_t)(j + u - k0) * w + q];
-        }
-#pragma unroll
-        for (int u = 0; u < PANEL_UF; ++u) v -= av[u] * wv[u];
-      }
-      for (; j < k; ++j) v -= A[(int64_t)j * r + i] * Wp[(int64_t)(j - k0) * w + q];
+      for (int u = 0; u < PANEL_UF; ++u) v -= av[u] * wv[u];
     }
+    for (; j < k; ++j) v -= A[(int64_t)j * r + i] * Wp[(int64_t)(j - k0) * w + q];
     return v;
   };
   int epoch = 0;
@@ -630,66 +588,18 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
     group_barrier(ctr, G, epoch, status);
     k += kstep;
   }
-  if (LDSP) {
-    // the staged columns back to the factor, and the W rows the trailing
-    // update reads (rows >= k of the eliminated columns)
-    for (int64_t e = threadIdx.x; e < (int64_t)(pc1 - k0) * (w - k0); e += 256) {
-      const int64_t j = e / (w - k0), i = e % (w - k0);
-      A[(k0 + j) * r + (k0 + i)] = As[j * ldsm + i];
-    }
-    for (int64_t e = threadIdx.x; e < (int64_t)(k - k0) * (w - k); e += 256) {
-      const int64_t j = e / (w - k), i = k + e % (w - k);
-      Wp[j * w + i] = Ws[j * ldsm + (i - k0)];
-    }
-  }
   if (gt == 0) {
     kstart[s] = k0;
     kpos[s] = k;
   }
 }
 
-// LDS of the staged panel of a diagonal block with up to `rows` rows
 template <typename T>
-size_t panel_lds(int rows) {
-  return sizeof(T) * (2 * (size_t)PANEL_NB + 2) * (size_t)rows;
-}
-template <typename T>
-int panel_lds_rows() {
-  return (int)(PANEL_LDS_BYTES / (sizeof(T) * (2 * (size_t)PANEL_NB + 2)));
-}
-template int panel_lds_rows<double>();
-template int panel_lds_rows<float>();
-
-template <typename T>
-void launch_bk_panel(const int* list, int count, int G, const SnArgs& a, T* valL, T* dval,
-                     int* perm_piv, T* W, const int64_t* woff, int* kpos, int* kstart, int* sync,
-                     int* status, bool cooperative, int lds_rows, hipStream_t st) {
+void launch_bk_panel(const int* list, int count, const SnArgs& a, T* valL, T* dval, int* perm_piv, T* W,
+                     const int64_t* woff, int* kpos, int* kstart, int* sync, int* status, hipStream_t st) {
   if (count <= 0) return;
-  if (lds_rows > 0) {
-    if (G != 1 || cooperative || lds_rows > panel_lds_rows<T>())
-      throw std::invalid_argument("bk_panel: LDS panel needs one workgroup per supernode and fitting rows");
-    static bool attr = false;
-    if (!attr) {
-      if (hipFuncSetAttribute((const void*)k_bk_panel<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)PANEL_LDS_BYTES) != hipSuccess)
-        throw std::runtime_error("bk_panel: LDS attribute");
-      attr = true;
-    }
-    k_bk_panel<T, true><<<count, 256, panel_lds<T>(lds_rows), st>>>(list, 1, a.super, a.pi, a.px, valL, dval,
-                                                                     perm_piv, W, woff, kpos, kstart, sync, a.n,
-                                                                     status, lds_rows);
-  } else if (!cooperative || G == 1) {
-    k_bk_panel<T, false><<<count * G, 256, 0, st>>>(list, G, a.super, a.pi, a.px, valL, dval, perm_piv, W, woff,
-                                                    kpos, kstart, sync, a.n, status, 0);
-  } else {
-    int n = a.n, z = 0;
-    void* args[] = {(void*)&list, (void*)&G, (void*)&a.super, (void*)&a.pi, (void*)&a.px,
-                    (void*)&valL, (void*)&dval, (void*)&perm_piv, (void*)&W, (void*)&woff,
-                    (void*)&kpos, (void*)&kstart, (void*)&sync, (void*)&n, (void*)&status, (void*)&z};
-    hipError_t e = hipLaunchCooperativeKernel((const void*)k_bk_panel<T, false>, dim3(count * G), dim3(256), args,
-                                              0, st);
-    if (e != hipSuccess) throw std::runtime_error(std::string("bk_panel coop: ") + hipGetErrorString(e));
-  }
+  k_bk_panel<T><<<count, 256, 0, st>>>(list, 1, a.super, a.pi, a.px, valL, dval, perm_piv, W, woff, kpos, kstart,
+                                       sync, a.n, status);
   HIP_LAUNCH_CHECK("bk_panel");
 }
 
@@ -2237,8 +2147,8 @@ void launch_k0(int n, int64_t nnzf, const int* rp, const int64_t* src, const dou
                                    const int*, const unsigned char*, hipStream_t);                             \
   template void launch_reset_supernodes<T>(const int*, int, const SnArgs&, T*, T*, int*, hipStream_t);          \
   template void launch_bk_small<T>(const int*, int, int, const SnArgs&, T*, T*, int*, int*, hipStream_t);      \
-  template void launch_bk_panel<T>(const int*, int, int, const SnArgs&, T*, T*, int*, T*, const int64_t*, int*, \
-                                   int*, int*, int*, bool, int, hipStream_t);                                       \
+  template void launch_bk_panel<T>(const int*, int, const SnArgs&, T*, T*, int*, T*, const int64_t*, int*, int*,  \
+                                   int*, int*, hipStream_t);                                       \
   template void launch_trailing<T>(const int*, int, int, int, const SnArgs&, T*, const T*, const int64_t*,      \
                                    const int*, const int*, hipStream_t);                                       \
   template void launch_offdiag<T>(const int*, int, int, const int*, const int*, int, const SnArgs&, T*,      \

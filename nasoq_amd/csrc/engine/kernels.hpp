@@ -8,7 +8,7 @@
 namespace lblg {
 
 constexpr int SMALL_W = 64;    // widest supernode factored entirely in LDS
-constexpr int PANEL_NB = 32;   // Bunch-Kaufman panel width for wider supernodes
+constexpr int PANEL_NB = 32;   // columns of a one-workgroup panel kept in memory
 constexpr int SOLVE_W = 128;   // column width of a solve piece
 constexpr int TRI_NARROW = 32; // triangle launches of a level: pieces up to this width, then the wider ones
 constexpr int MAX_RHS = 8;     // right-hand sides per solve call
@@ -51,16 +51,10 @@ void launch_scatter_values(int64_t count, const int64_t* idx, const double* vals
 template <typename T>
 void launch_bk_small(const int* list, int count, int wmax, const SnArgs& a, T* valL, T* dval,
                      int* perm_piv, int* status, hipStream_t st);
-// lds_rows > 0: one workgroup per supernode with the panel staged in LDS
-// (every supernode of the list has at most lds_rows <= panel_lds_rows<T>()
-// columns); 0: the panel stays in memory
-constexpr size_t PANEL_LDS_BYTES = 150 * 1024;
+// one workgroup per listed supernode, panels of PANEL_NB columns in memory
 template <typename T>
-int panel_lds_rows();
-template <typename T>
-void launch_bk_panel(const int* list, int count, int G, const SnArgs& a, T* valL, T* dval,
-                     int* perm_piv, T* W, const int64_t* woff, int* kpos, int* kstart, int* sync,
-                     int* status, bool cooperative, int lds_rows, hipStream_t st);
+void launch_bk_panel(const int* list, int count, const SnArgs& a, T* valL, T* dval, int* perm_piv, T* W,
+                     const int64_t* woff, int* kpos, int* kstart, int* sync, int* status, hipStream_t st);
 // wide panels with flag-in-word exchange (bk_wide.hip)
 constexpr int WIDE_NB = 64;         // panel width
 constexpr int WIDE_ROWS = 192;      // far rows per workgroup (256-thread workgroups)
@@ -71,6 +65,11 @@ constexpr int WIDE_MOVED = 128;     // moved indices per panel (scratch rows)
 // columns of a 256-byte LDS row (32 FP64, 64 FP32)
 inline int wide_panel_nb(int nt, size_t value_size) { return nt == 256 ? 64 : (value_size == 8 ? 32 : 64); }
 constexpr int64_t LL_WORDS = 2 * 256 * 4 + 2 * 256 * 8 + 2 * 256 * 2 * 64;
+struct PanelList {  // supernodes of a one-workgroup panel launch, one per workgroup
+  const int* list;
+  const int* super;
+  const int64_t *pi, *px, *woff;
+};
 struct WideSn {  // one wide supernode: first column, width, rows, offsets of its panel and workspace
   int s, c0, w;
   int64_t r, px, woff;
@@ -79,6 +78,15 @@ template <typename T>
 void launch_bk_wide(const WideSn& sn, int G, int nt, int nb, int sub, int wcols, int n, T* valL, T* dval,
                     int* perm_piv, T* W, int* kpos, int* kstart, int* sync, int* sync_next, uint64_t* ll,
                     uint32_t ebase, int* status, hipStream_t st);
+// One-workgroup panels of the listed supernodes, all with at most `rows`
+// diagonal-block rows left: one_panel_nb<T>(rows) columns each (0: too many
+// rows; those take launch_bk_panel).
+constexpr int ONE_WCOLS = 64;  // columns of their W workspace
+template <typename T>
+int one_panel_nb(int rows);
+template <typename T>
+void launch_bk_one(const int* list, int count, int rows, const SnArgs& a, T* valL, T* dval, int* perm_piv, T* W,
+                   const int64_t* woff, int* kpos, int* kstart, int* status, hipStream_t st);
 template <typename T>
 void launch_trailing(const int* list, int count, int tiles_per_sn, int lo, const SnArgs& a, T* valL,
                      const T* W, const int64_t* woff, const int* kpos, const int* kstart,
