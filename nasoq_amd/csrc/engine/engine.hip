@@ -1288,9 +1288,6 @@ void factor(Handle& h) {
     h.values_dirty = true;
   }
   DeviceFactor& D = *h.dev;
-  double md = 0.0;
-  for (double v : h.Ax) md = std::max(md, std::fabs(v));
-  h.max_abs_entry = md;
   // a restricted refactorization updates the device factor of the values
   // last uploaded (same precision and perturbation settings) after
   // lblg_update_values changes; the FP32 / BF16 factors keep the diagonal
@@ -1497,8 +1494,9 @@ void apply_solve(DeviceFactor& D, const double* in, double* out, int nrhs, const
     apply_solve_t<double>(D, in, out, nrhs, active, astride);
 }
 
-static void spmv_ordered(DeviceFactor& D, const double* x, double* y, int nrhs) {
-  timed(D, "spmv", [&] { launch_spmv(D.n, D.Krp, D.Kci, D.Kv, D.perm_f, D.iperm_f, x, y, nrhs, D.stream); });
+// y = K0 x, or b - K0 x
+static void spmv_ordered(DeviceFactor& D, const double* x, double* y, int nrhs, const double* b = nullptr) {
+  timed(D, "spmv", [&] { launch_spmv(D.n, D.Krp, D.Kci, D.Kv, D.perm_f, D.iperm_f, x, b, y, nrhs, D.stream); });
 }
 
 
@@ -1514,9 +1512,17 @@ static void gmres_cycle(DeviceFactor& D, const double* b, double* x, int nrhs, i
   double* coef0 = D.gm + gmres_off_D(MR);
   double* reo = D.gm + gmres_off_D(MR) + 1;
   auto Vk = [&](int k) { return D.V + (int64_t)k * nn; };
-  spmv_ordered(D, x, D.T, nrhs);
-  launch_sub(nn, b, D.T, D.R, st);
+  spmv_ordered(D, x, D.R, nrhs, b);
   apply_solve(D, D.R, D.Xs, nrhs, nullptr, 0);
+  if (gmres_one(n, nrhs) && mr <= MR) {
+    launch_gmres_begin(n, nrhs, MR, D.gm, D.Xs, D.V, itr, tol_abs, tol_rel, st);
+    for (int k = 0; k < mr; ++k) {
+      spmv_ordered(D, Vk(k), D.T, nrhs);
+      apply_solve(D, D.T, Vk(k + 1), nrhs, mask, SS);  // columns out of the step keep V(k + 1) = 0
+      launch_gmres_step(n, nrhs, MR, mr, k, D.gm, D.V, x, itr, tol_abs, tol_rel, st);
+    }
+    return;
+  }
   launch_dot_scalar(n, nrhs, D.Xs, D.Xs, D.part, D.nblk_red, D.dots, 0, MR, D.gm, 0, 0,
                     itr, tol_abs, tol_rel, st);
   launch_fill(D.V, nn * (MR + 1), 0.0, st);
@@ -1551,9 +1557,7 @@ static void gmres_cycle(DeviceFactor& D, const double* b, double* x, int nrhs, i
 // ||b - K0 x||_1 / (||K0||_inf ||x||_1 + ||b||_1)
 static void backward_errors(Handle& h, const double* b, const double* x, int nrhs, double* err) {
   DeviceFactor& D = *h.dev;
-  const int64_t nn = (int64_t)D.n * nrhs;
-  spmv_ordered(D, x, D.T, nrhs);
-  launch_sub(nn, b, D.T, D.R, D.stream);
+  spmv_ordered(D, x, D.R, nrhs, b);
   if (D.nseg > 0) {
     // a block-diagonal batch: every system's own backward error, the worst per column
     // (the systems occupy the same contiguous row ranges in both orderings)

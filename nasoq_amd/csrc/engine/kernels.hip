@@ -20,6 +20,7 @@
 #include <cstdio>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 #include "engine/kernels.hpp"
 #include "engine/device_util.hpp"
@@ -1589,8 +1590,9 @@ void launch_bwd_tri(const int* pieces, int np, int maxpw, const int* piece_sn, c
 // --------------------------------------------------------------------------
 // y_ord = P K0 P^T x_ord with the full CSR of K0 in the original ordering
 // --------------------------------------------------------------------------
+// (y_ord = b_ord - P K0 P^T x_ord when b is given: the residual in one launch)
 __global__ void k_spmv(int n, const int* rp, const int* ci, const double* v, const int* perm_f,
-                       const int* iperm_f, const double* x, double* y, int nrhs) {
+                       const int* iperm_f, const double* x, const double* b, double* y, int nrhs) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int row = perm_f[i];
     double acc[MAXRHS];
@@ -1600,12 +1602,13 @@ __global__ void k_spmv(int n, const int* rp, const int* ci, const double* v, con
       const int j = iperm_f[ci[q]];
       for (int c = 0; c < nrhs; ++c) acc[c] += a * x[(int64_t)j * nrhs + c];
     }
-    for (int c = 0; c < nrhs; ++c) y[(int64_t)i * nrhs + c] = acc[c];
+    for (int c = 0; c < nrhs; ++c)
+      y[(int64_t)i * nrhs + c] = b ? b[(int64_t)i * nrhs + c] - acc[c] : acc[c];
   }
 }
 void launch_spmv(int n, const int* rp, const int* ci, const double* v, const int* perm_f, const int* iperm_f,
-                 const double* x, double* y, int nrhs, hipStream_t st) {
-  k_spmv<<<grid_for(n, 256), 256, 0, st>>>(n, rp, ci, v, perm_f, iperm_f, x, y, nrhs);
+                 const double* x, const double* b, double* y, int nrhs, hipStream_t st) {
+  k_spmv<<<grid_for(n, 256), 256, 0, st>>>(n, rp, ci, v, perm_f, iperm_f, x, b, y, nrhs);
   HIP_LAUNCH_CHECK("spmv");
 }
 
@@ -1887,43 +1890,223 @@ void launch_gmres_scalar(int op, int nrhs, int MR, double* gm, const double* dot
   HIP_LAUNCH_CHECK("gmres_scalar");
 }
 
-// dot products of short vectors followed by the GMRES scalar step on them,
-// in one workgroup and one launch (launch_dot + launch_gmres_scalar for long
-// vectors); the sums are those of k_dot_one
-__global__ __launch_bounds__(1024) void k_dot_scalar_one(int n, int nrhs, const double* a, const double* b,
-                                                         double* out, int op, int MR, double* gm, int j, int k,
-                                                         int itr, double tol_abs, double tol_rel) {
-  __shared__ double sh[16][MAXRHS];
+// --------------------------------------------------------------------------
+// The vector work of GMRES on short vectors (rows x columns up to
+// DOT_ONE_MAX) in one workgroup: k_gmres_begin after the preconditioned
+// residual, k_gmres_step after each preconditioned basis vector.  Launch by
+// launch (a dot product with its scalar step, an update, ...) an inner step
+// took 4 k + 9 launches of about 4 us and 2 us between them, 0.9 ms of the
+// 3 ms that an active-set iteration of the 40 x 40 QP takes with its nine
+// inner steps.  An update and the dot product after it share a pass over the
+// vectors.  The sums are k_dot_one's: strided per-thread sums (thread t has
+// rows t, t + 1024, ...), then a fixed tree, so repeated calls agree bit for
+// bit.  The columns' state is worked on in LDS (GM_LDS doubles hold it for
+// restart lengths up to 16; beyond, in memory).
+// --------------------------------------------------------------------------
+// f(std::integral_constant<int, nrhs>) for 1 <= nrhs <= MAXRHS
+template <typename F>
+static void with_nrhs(int nrhs, F f) {
+  switch (nrhs) {
+    case 1: f(std::integral_constant<int, 1>()); return;
+    case 2: f(std::integral_constant<int, 2>()); return;
+    case 3: f(std::integral_constant<int, 3>()); return;
+    case 4: f(std::integral_constant<int, 4>()); return;
+    case 5: f(std::integral_constant<int, 5>()); return;
+    case 6: f(std::integral_constant<int, 6>()); return;
+    case 7: f(std::integral_constant<int, 7>()); return;
+    case 8: f(std::integral_constant<int, 8>()); return;
+  }
+  throw std::invalid_argument("right-hand sides out of range");
+}
+constexpr int GM_LDS = MAXRHS * (17 * 16 + 4 * 17 + 18 + 8);
+struct GmresState {
+  double* gm;  // where the state is worked on
+  bool lds;
+};
+template <int NR>
+__device__ inline GmresState gm_open(double* gm, int MR, double* lds) {
+  const int total = NR * ((MR + 1) * MR + 4 * (MR + 1) + (MR + 2) + 8);
+  if (total > GM_LDS) return {gm, false};
+  for (int i = threadIdx.x; i < total; i += 1024) lds[i] = gm[i];
+  __syncthreads();
+  return {lds, true};
+}
+template <int NR>
+__device__ inline void gm_close(const GmresState& G, double* gm, int MR) {
+  if (!G.lds) return;
+  __syncthreads();
+  const int total = NR * ((MR + 1) * MR + 4 * (MR + 1) + (MR + 2) + 8);
+  for (int i = threadIdx.x; i < total; i += 1024) gm[i] = G.gm[i];
+}
+// column sums over the workgroup, then the scalar step `op` on them
+template <int NR>
+__device__ inline void gm_reduce(const double* acc, double (*sh)[NR], int op, const GmresState& G, int MR, int j,
+                                 int k, int itr, double tol_abs, double tol_rel) {
   const int t = threadIdx.x, wv = t >> 6, ln = t & 63;
-  double acc[MAXRHS];
 #pragma unroll
-  for (int c = 0; c < MAXRHS; ++c) acc[c] = 0.0;
-  for (int i = t; i < n; i += 1024)
-#pragma unroll
-    for (int c = 0; c < MAXRHS; ++c)
-      if (c < nrhs) acc[c] += a[(int64_t)i * nrhs + c] * b[(int64_t)i * nrhs + c];
-#pragma unroll
-  for (int c = 0; c < MAXRHS; ++c) {
-    if (c >= nrhs) break;
+  for (int c = 0; c < NR; ++c) {
     const double v = wave_sum(acc[c]);
     if (ln == 0) sh[wv][c] = v;
   }
   __syncthreads();
-  if (t < nrhs) {
+  if (t < NR) {
     double s = 0.0;
+#pragma unroll
     for (int q = 0; q < 16; ++q) s += sh[q][t];
-    out[t] = s;
-    gmres_scalar_col(op, t, MR, gm, s, j, k, itr, tol_abs, tol_rel);
+    gmres_scalar_col(op, t, MR, G.gm, s, j, k, itr, tol_abs, tol_rel);
+    if (!G.lds) __threadfence_block();
   }
+  __syncthreads();
 }
+
+// V(0) = z / ||z|| for the running columns (z the preconditioned residual),
+// V(1..MR) = 0
+template <int NR>
+__global__ __launch_bounds__(1024) void k_gmres_begin(int n, int MR, double* gm, const double* z, double* V, int itr,
+                                                      double tol_abs, double tol_rel) {
+  __shared__ double sh[16][NR];
+  __shared__ double gl[GM_LDS];
+  const GmresState G = gm_open<NR>(gm, MR, gl);
+  double acc[NR];
+#pragma unroll
+  for (int c = 0; c < NR; ++c) acc[c] = 0.0;
+  for (int i = threadIdx.x; i < n; i += 1024)
+#pragma unroll
+    for (int c = 0; c < NR; ++c) {
+      const double v = z[(int64_t)i * NR + c];
+      acc[c] += v * v;
+    }
+  gm_reduce<NR>(acc, sh, 0, G, MR, 0, 0, itr, tol_abs, tol_rel);
+  double rho[NR];
+#pragma unroll
+  for (int c = 0; c < NR; ++c) {
+    double* st = gs_col(G.gm, c, MR);
+    rho[c] = GS_S(st, MR)[7] != 0.0 ? GS_D(st, MR)[0] : 0.0;
+  }
+  const int64_t nn = (int64_t)n * NR;
+  for (int i = threadIdx.x; i < n; i += 1024)
+#pragma unroll
+    for (int c = 0; c < NR; ++c) {
+      const int64_t e = (int64_t)i * NR + c;
+      V[e] = rho[c] != 0.0 ? z[e] / rho[c] : 0.0;
+    }
+  for (int64_t e = nn + threadIdx.x; e < nn * (MR + 1); e += 1024) V[e] = 0.0;
+  gm_close<NR>(G, gm, MR);
+}
+
+// inner step k on w = V(k + 1) = M^-1 K V(k): modified Gram-Schmidt, the
+// conditional re-orthogonalisation, w / ||w||, the Givens rotation; after
+// the last step (k + 1 == mr) the least-squares solution and x += V y
+template <int NR>
+__global__ __launch_bounds__(1024) void k_gmres_step(int n, int MR, int mr, int k, double* gm, double* V, double* x,
+                                                     int itr, double tol_abs, double tol_rel) {
+  __shared__ double sh[16][NR];
+  __shared__ double gl[GM_LDS];
+  const GmresState G = gm_open<NR>(gm, MR, gl);
+  const int64_t nn = (int64_t)n * NR;
+  double* w = V + (k + 1) * nn;
+  double acc[NR], co[NR];
+  bool on[NR], any = false;
+#pragma unroll
+  for (int c = 0; c < NR; ++c) {
+    on[c] = GS_S(gs_col(G.gm, c, MR), MR)[7] != 0.0;
+    any = any || on[c];
+  }
+  if (any) {
+    // w -= co u for the columns that are on (u: none when null), and the
+    // column sums of w . q (q: w itself when null)
+    auto pass = [&](const double* u, const double* q) {
+#pragma unroll
+      for (int c = 0; c < NR; ++c) acc[c] = 0.0;
+      for (int i = threadIdx.x; i < n; i += 1024)
+#pragma unroll
+        for (int c = 0; c < NR; ++c) {
+          const int64_t e = (int64_t)i * NR + c;
+          double v = w[e];
+          if (u && on[c]) {
+            v -= co[c] * u[e];
+            w[e] = v;
+          }
+          acc[c] += v * (q ? q[e] : v);
+        }
+    };
+    auto coefs = [&]() {
+#pragma unroll
+      for (int c = 0; c < NR; ++c) co[c] = GS_D(gs_col(G.gm, c, MR), MR)[0];
+    };
+    pass(nullptr, nullptr);
+    gm_reduce<NR>(acc, sh, 1, G, MR, 0, k, itr, tol_abs, tol_rel);
+    pass(nullptr, V);
+    gm_reduce<NR>(acc, sh, 2, G, MR, 0, k, itr, tol_abs, tol_rel);
+    for (int j = 0; j <= k; ++j) {
+      coefs();
+      pass(V + j * nn, j < k ? V + (j + 1) * nn : nullptr);
+      gm_reduce<NR>(acc, sh, j < k ? 2 : 3, G, MR, j + 1, k, itr, tol_abs, tol_rel);
+    }
+    bool run[NR], reo = false;  // conditional re-orthogonalisation
+#pragma unroll
+    for (int c = 0; c < NR; ++c) {
+      run[c] = on[c];
+      on[c] = GS_D(gs_col(G.gm, c, MR), MR)[1] != 0.0;
+      reo = reo || on[c];
+    }
+    if (reo) {
+      pass(nullptr, V);
+      gm_reduce<NR>(acc, sh, 4, G, MR, 0, k, itr, tol_abs, tol_rel);
+      for (int j = 0; j <= k; ++j) {
+        coefs();
+        pass(V + j * nn, j < k ? V + (j + 1) * nn : nullptr);
+        gm_reduce<NR>(acc, sh, j < k ? 4 : 5, G, MR, j + 1, k, itr, tol_abs, tol_rel);
+      }
+    }
+    coefs();
+    for (int i = threadIdx.x; i < n; i += 1024)
+#pragma unroll
+      for (int c = 0; c < NR; ++c)
+        if (run[c] && co[c] != 0.0) w[(int64_t)i * NR + c] /= co[c];
+    __syncthreads();  // the coefficients are read: the state may change
+    if (threadIdx.x < NR) gmres_scalar_col(6, threadIdx.x, MR, G.gm, 0.0, 0, k, itr, tol_abs, tol_rel);
+  }
+  if (k + 1 == mr) {
+    if (threadIdx.x < NR) {
+      gmres_scalar_col(7, threadIdx.x, MR, G.gm, 0.0, 0, 0, itr, tol_abs, tol_rel);
+      if (!G.lds) __threadfence_block();
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += 1024)
+#pragma unroll
+      for (int c = 0; c < NR; ++c) {
+        const double* y = GS_Y(gs_col(G.gm, c, MR), MR);
+        double v = x[(int64_t)i * NR + c];
+        for (int j = 0; j <= MR; ++j)
+          if (y[j] != 0.0) v += V[((int64_t)j * n + i) * NR + c] * y[j];
+        x[(int64_t)i * NR + c] = v;
+      }
+  }
+  gm_close<NR>(G, gm, MR);
+}
+bool gmres_one(int n, int nrhs) { return (int64_t)n * nrhs <= DOT_ONE_MAX; }
+void launch_gmres_begin(int n, int nrhs, int MR, double* gm, const double* z, double* V, int itr, double tol_abs,
+                        double tol_rel, hipStream_t st) {
+  auto go = [&](auto nr) {
+    k_gmres_begin<decltype(nr)::value><<<1, 1024, 0, st>>>(n, MR, gm, z, V, itr, tol_abs, tol_rel);
+  };
+  with_nrhs(nrhs, go);
+  HIP_LAUNCH_CHECK("gmres_begin");
+}
+void launch_gmres_step(int n, int nrhs, int MR, int mr, int k, double* gm, double* V, double* x, int itr,
+                       double tol_abs, double tol_rel, hipStream_t st) {
+  auto go = [&](auto nr) {
+    k_gmres_step<decltype(nr)::value><<<1, 1024, 0, st>>>(n, MR, mr, k, gm, V, x, itr, tol_abs, tol_rel);
+  };
+  with_nrhs(nrhs, go);
+  HIP_LAUNCH_CHECK("gmres_step");
+}
+
+// a dot product and the scalar step on it (long vectors)
 void launch_dot_scalar(int n, int nrhs, const double* a, const double* b, double* part, int nblk, double* out,
                        int op, int MR, double* gm, int j, int k, int itr, double tol_abs, double tol_rel,
                        hipStream_t st) {
-  if ((int64_t)n * nrhs <= DOT_ONE_MAX) {
-    k_dot_scalar_one<<<1, 1024, 0, st>>>(n, nrhs, a, b, out, op, MR, gm, j, k, itr, tol_abs, tol_rel);
-    HIP_LAUNCH_CHECK("dot_scalar");
-    return;
-  }
   launch_dot(n, nrhs, a, b, part, nblk, out, st);
   launch_gmres_scalar(op, nrhs, MR, gm, out, j, k, itr, tol_abs, tol_rel, st);
 }

@@ -145,7 +145,15 @@ template <typename T>
 void launch_bwd_chain(int s, int w, int64_t r, const SnArgs& a, const T* valL, const T* Z, T* offacc, T* Xf,
                       int nrhs, uint64_t* xb, uint32_t epoch, int* status, hipStream_t st);
 void launch_spmv(int n, const int* rp, const int* ci, const double* v, const int* perm_f, const int* iperm_f,
-                 const double* x, double* y, int nrhs, hipStream_t st);
+                 const double* x, const double* b, double* y, int nrhs, hipStream_t st);
+// GMRES vector work of short vectors in one workgroup (gmres_one: whether
+// n x nrhs is short): after the preconditioned residual z, and after inner
+// step k's preconditioned basis vector in V(k + 1)
+bool gmres_one(int n, int nrhs);
+void launch_gmres_begin(int n, int nrhs, int MR, double* gm, const double* z, double* V, int itr, double tol_abs,
+                        double tol_rel, hipStream_t st);
+void launch_gmres_step(int n, int nrhs, int MR, int mr, int k, double* gm, double* V, double* x, int itr,
+                       double tol_abs, double tol_rel, hipStream_t st);
 void launch_gather_rhs(int n, int nrhs, const double* B, int64_t ldb, const int* perm_f, double* out,
                        hipStream_t st);
 void launch_scatter_sol(int n, int nrhs, const double* Xo, const int* perm_f, double* X, int64_t ldx,
