@@ -109,19 +109,110 @@ static void gemm(int M, int N, int K, const TA* A, int64_t sa0, int64_t sa1, con
   HIP_LAUNCH_CHECK("gemm_bf16");
 }
 
-// Z(b, j) += bias(j), then ReLU in place when relu != 0
-__global__ void k_bias_act(float* Z, const float* bias, int rows, int cols, int relu) {
-  const int64_t n = (int64_t)rows * cols;
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
-    float v = Z[q] + bias[q % cols];
-    Z[q] = (relu && v < 0.f) ? 0.f : v;
+// --------------------------------------------------------------------------
+// The products with a weight matrix: C(i, j) = f(sum_k A(i, k) W(k, j)), A
+// FP32 with k contiguous (rounded to BF16 as it is read), W the BF16 copy,
+// W(k, j) = W[k sw0 + j sw1] with one of the strides 1.  A minibatch has few
+// rows, so 64 x 64 tiles gave 16 workgroups on 256 CUs and a chain of K / 32
+// staged chunks, 62 us at 64 x 1024 x 1024.  Here a workgroup has a 32 x 32
+// tile (64 workgroups there), its four waves take every fourth 16-deep slice
+// of k with operands loaded lane by lane, several slices in flight, and meet
+// in LDS in a fixed order: 11 us.  f: bias (added when given), ReLU, or the
+// mask dA(i, j) = 0 where act(i, j) <= 0 of the backward pass, so that no
+// separate pass follows.
+// --------------------------------------------------------------------------
+enum { EPI_NONE = 0, EPI_RELU = 1, EPI_MASK = 2 };
+constexpr int WT = 32;  // output tile
+// four consecutive k of A's row, zero beyond K
+template <bool VEC>
+__device__ inline s4 load_a(const float* row, int k, int K) {
+  float v[4];
+  if (VEC) {  // K and the rows are multiples of four
+    const f4 x = k < K ? *reinterpret_cast<const f4*>(row + k) : f4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 4; ++e) v[e] = x[e];
+  } else {
+    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? row[k + e] : 0.f;
+  }
+  s4 r;
+  for (int e = 0; e < 4; ++e) r[e] = (short)f2bf(v[e]);
+  return r;
+}
+template <bool VEC>
+__device__ inline s4 load_w(const unsigned short* col, int64_t sw0, int k, int K) {
+  if (VEC && sw0 == 1) return k < K ? *reinterpret_cast<const s4*>(col + k) : s4{0, 0, 0, 0};
+  s4 r;
+  for (int e = 0; e < 4; ++e) r[e] = k + e < K ? (short)col[(int64_t)(k + e) * sw0] : (short)0;
+  return r;
+}
+template <bool VEC>
+__global__ __launch_bounds__(256) void k_gemm_weight(int M, int N, int K, const float* A, int lda,
+                                                     const unsigned short* W, int64_t sw0, int64_t sw1, float* C,
+                                                     int ldc, const float* bias, const float* act, int epi) {
+  __shared__ float red[4][WT][WT + 1];
+  const int t = threadIdx.x, wv = t >> 6, ln = t & 63, li = ln & 15, lk = 4 * (ln >> 4);
+  const int i0 = blockIdx.y * WT, j0 = blockIdx.x * WT;
+  // rows and columns beyond the matrix read the last one and are not stored
+  const float* ar[2];
+  const unsigned short* wc[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    ar[r] = A + (int64_t)min(i0 + 16 * r + li, M - 1) * lda;
+    wc[r] = W + (int64_t)min(j0 + 16 * r + li, N - 1) * sw1;
+  }
+  f4 acc[2][2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[r][c] = f4{0.f, 0.f, 0.f, 0.f};
+  constexpr int U = 4;  // slices in flight
+  for (int k0 = 16 * wv; k0 < K; k0 += 64 * U) {
+    s4 a[U][2], b[U][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        a[u][r] = load_a<VEC>(ar[r], k0 + 64 * u + lk, K);
+        b[u][r] = load_w<VEC>(wc[r], sw0, k0 + 64 * u + lk, K);
+      }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[u][r], b[u][c], acc[r][c], 0, 0, 0);
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[wv][16 * r + lk + e][16 * c + li] = acc[r][c][e];
+  __syncthreads();
+  for (int q = t; q < WT * WT; q += 256) {
+    const int i = q / WT, j = q % WT;
+    if (i0 + i < M && j0 + j < N) {
+      float v = (red[0][i][j] + red[1][i][j]) + (red[2][i][j] + red[3][i][j]);
+      if (bias) v += bias[j0 + j];
+      if (epi == EPI_RELU && v < 0.f) v = 0.f;
+      if (epi == EPI_MASK && !(act[(int64_t)(i0 + i) * ldc + j0 + j] > 0.f)) v = 0.f;
+      C[(int64_t)(i0 + i) * ldc + j0 + j] = v;
+    }
   }
 }
-// dA *= (A > 0)
-__global__ void k_relu_back(float* dA, const float* A, int64_t n) {
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x)
-    if (!(A[q] > 0.f)) dA[q] = 0.f;
+static void gemm_weight(int M, int N, int K, const float* A, const unsigned short* W, int64_t sw0, int64_t sw1,
+                        float* C, const float* bias, const float* act, int epi, hipStream_t st) {
+  const dim3 grid((N + WT - 1) / WT, (M + WT - 1) / WT);
+  // four-element loads: rows of A (and of W, read along k) on their alignment
+  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
+                   (sw0 != 1 || (sw1 % 4 == 0 && reinterpret_cast<uintptr_t>(W) % 8 == 0));
+  if (vec)
+    k_gemm_weight<true><<<grid, 256, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, bias, act, epi);
+  else
+    k_gemm_weight<false><<<grid, 256, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, bias, act, epi);
+  HIP_LAUNCH_CHECK("gemm_weight");
 }
+
 // logits Z, labels Y (n = batch x out entries): dZ = (sigmoid(Z) - Y) / n and
 // loss += the mean of the stable BCE terms max(z, 0) - z y + log(1 + e^-|z|)
 __global__ void k_bce(const float* Z, const float* Y, int64_t n, float* dZ, float* loss) {
@@ -143,13 +234,22 @@ __global__ void k_sigmoid(const float* Z, float* P, int64_t n) {
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x)
     P[q] = 1.f / (1.f + expf(-Z[q]));
 }
-// db(j) = sum_b dZ(b, j)
-__global__ void k_colsum(const float* dZ, int rows, int cols, float* db) {
-  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < cols; j += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int b = 0; b < rows; ++b) s += dZ[(int64_t)b * cols + j];
-    db[j] = s;
+// db(j) = sum_b dZ(b, j): 64 columns a workgroup, its four waves take every
+// fourth row, a fixed order
+__global__ __launch_bounds__(256) void k_colsum(const float* dZ, int rows, int cols, float* db) {
+  __shared__ float sh[4][64];
+  const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63, j = blockIdx.x * 64 + ln;
+  float s = 0.f;
+  if (j < cols) {
+#pragma unroll 8
+    for (int b = wv; b < rows; b += 4) s += dZ[(int64_t)b * cols + j];
   }
+  sh[wv][ln] = s;
+  __syncthreads();
+  if (wv == 0 && j < cols) db[j] = (sh[0][ln] + sh[1][ln]) + (sh[2][ln] + sh[3][ln]);
+}
+static void colsum(const float* dZ, int rows, int cols, float* db, hipStream_t st) {
+  k_colsum<<<(cols + 63) / 64, 256, 0, st>>>(dZ, rows, cols, db);
 }
 // Adam (Kingma & Ba 2015) on the FP32 master parameters, then their BF16 copy
 __global__ void k_adam(float* P, unsigned short* Pb, const float* G, float* Mo, float* Vo, int64_t n, float lr,
@@ -215,12 +315,9 @@ struct Mlp {
     if (st) (void)hipStreamDestroy(st);
   }
   void forward(int B) {
-    gemm(B, h1, in, X, in, 1, Pb + oW1, 1, in, A1, h1, st);
-    k_bias_act<<<ew_grid((int64_t)B * h1), 256, 0, st>>>(A1, P + ob1, B, h1, 1);
-    gemm(B, h2, h1, A1, h1, 1, Pb + oW2, 1, h1, A2, h2, st);
-    k_bias_act<<<ew_grid((int64_t)B * h2), 256, 0, st>>>(A2, P + ob2, B, h2, 1);
-    gemm(B, out, h2, A2, h2, 1, Pb + oW3, 1, h2, Z3, out, st);
-    k_bias_act<<<ew_grid((int64_t)B * out), 256, 0, st>>>(Z3, P + ob3, B, out, 0);
+    gemm_weight(B, h1, in, X, Pb + oW1, 1, in, A1, P + ob1, nullptr, EPI_RELU, st);
+    gemm_weight(B, h2, h1, A1, Pb + oW2, 1, h1, A2, P + ob2, nullptr, EPI_RELU, st);
+    gemm_weight(B, out, h2, A2, Pb + oW3, 1, h2, Z3, P + ob3, nullptr, EPI_NONE, st);
     HIP_LAUNCH_CHECK("mlp forward");
   }
   // gradients of the mean BCE over the batch into G; loss into *loss (device)
@@ -229,15 +326,13 @@ struct Mlp {
     const int64_t no = (int64_t)B * out;
     k_bce<<<ew_grid(no), 256, 0, st>>>(Z3, Y, no, dZ3, loss);
     gemm(out, h2, B, dZ3, 1, out, A2, h2, 1, G + oW3, h2, st);  // dW3 = dZ3^T A2
-    k_colsum<<<ew_grid(out), 256, 0, st>>>(dZ3, B, out, G + ob3);
-    gemm(B, h2, out, dZ3, out, 1, Pb + oW3, h2, 1, dA2, h2, st);  // dA2 = dZ3 W3
-    k_relu_back<<<ew_grid((int64_t)B * h2), 256, 0, st>>>(dA2, A2, (int64_t)B * h2);
+    colsum(dZ3, B, out, G + ob3, st);
+    gemm_weight(B, h2, out, dZ3, Pb + oW3, h2, 1, dA2, nullptr, A2, EPI_MASK, st);  // dA2 = dZ3 W3 where A2 > 0
     gemm(h2, h1, B, dA2, 1, h2, A1, h1, 1, G + oW2, h1, st);  // dW2 = dA2^T A1
-    k_colsum<<<ew_grid(h2), 256, 0, st>>>(dA2, B, h2, G + ob2);
-    gemm(B, h1, h2, dA2, h2, 1, Pb + oW2, h1, 1, dA1, h1, st);  // dA1 = dA2 W2
-    k_relu_back<<<ew_grid((int64_t)B * h1), 256, 0, st>>>(dA1, A1, (int64_t)B * h1);
+    colsum(dA2, B, h2, G + ob2, st);
+    gemm_weight(B, h1, h2, dA2, Pb + oW2, h1, 1, dA1, nullptr, A1, EPI_MASK, st);  // dA1 = dA2 W2 where A1 > 0
     gemm(h1, in, B, dA1, 1, h1, X, in, 1, G + oW1, in, st);  // dW1 = dA1^T X
-    k_colsum<<<ew_grid(h1), 256, 0, st>>>(dA1, B, h1, G + ob1);
+    colsum(dA1, B, h1, G + ob1, st);
     HIP_LAUNCH_CHECK("mlp backward");
   }
   void adam(float lr) {
