@@ -1496,7 +1496,7 @@ void apply_solve(DeviceFactor& D, const double* in, double* out, int nrhs, const
 
 // y = K0 x, or b - K0 x
 static void spmv_ordered(DeviceFactor& D, const double* x, double* y, int nrhs, const double* b = nullptr) {
-  timed(D, "spmv", [&] { launch_spmv(D.n, D.Krp, D.Kci, D.Kv, D.perm_f, D.iperm_f, x, b, y, nrhs, D.stream); });
+  timed(D, "spmv", [&] { launch_spmv(D.n, D.nnzf, D.Krp, D.Kci, D.Kv, D.perm_f, D.iperm_f, x, b, y, nrhs, D.stream); });
 }
 
 

@@ -1606,9 +1606,55 @@ __global__ void k_spmv(int n, const int* rp, const int* ci, const double* v, con
       y[(int64_t)i * nrhs + c] = b ? b[(int64_t)i * nrhs + c] - acc[c] : acc[c];
   }
 }
-void launch_spmv(int n, const int* rp, const int* ci, const double* v, const int* perm_f, const int* iperm_f,
-                 const double* x, const double* b, double* y, int nrhs, hipStream_t st) {
-  k_spmv<<<grid_for(n, 256), 256, 0, st>>>(n, rp, ci, v, perm_f, iperm_f, x, b, y, nrhs);
+// the same with L adjacent lanes per row (rows of many entries: one thread's
+// serial chain of gathers would set the time)
+template <int L>
+__global__ __launch_bounds__(256) void k_spmv_lanes(int n, const int* rp, const int* ci, const double* v,
+                                                    const int* perm_f, const int* iperm_f, const double* x,
+                                                    const double* b, double* y, int nrhs) {
+  const int sub = threadIdx.x % L;
+  for (int i = (blockIdx.x * blockDim.x + threadIdx.x) / L; i < n; i += gridDim.x * blockDim.x / L) {
+    const int row = perm_f[i], q1 = rp[row + 1];
+    double acc[MAXRHS];
+#pragma unroll
+    for (int c = 0; c < MAXRHS; ++c) acc[c] = 0.0;
+    for (int q = rp[row] + sub; q < q1; q += L) {
+      const double a = v[q];
+      const double* xj = x + (int64_t)iperm_f[ci[q]] * nrhs;
+#pragma unroll
+      for (int c = 0; c < MAXRHS; ++c)
+        if (c < nrhs) acc[c] += a * xj[c];
+    }
+#pragma unroll
+    for (int c = 0; c < MAXRHS; ++c) {
+      if (c >= nrhs) break;
+      double s = acc[c];
+#pragma unroll
+      for (int o = L / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (sub == 0) {
+        const int64_t e = (int64_t)i * nrhs + c;
+        y[e] = b ? b[e] - s : s;
+      }
+    }
+  }
+}
+void launch_spmv(int n, int64_t nnz, const int* rp, const int* ci, const double* v, const int* perm_f,
+                 const int* iperm_f, const double* x, const double* b, double* y, int nrhs, hipStream_t st) {
+  // Lanes per row by the mean entries per row; one thread per row before,
+  // now (us, one / four right-hand sides): mean 236, n = 3600: 197 / 267 -> 9.4 /
+  // 13.8; 101: 88 / 86 -> 7.5 / 9.9; 51: 38 / 47 -> 7.4 / 8.4; 25: 17 / 27 -> 6.6 /
+  // 7.6; 12: 11 / 17 -> 6.8 / 7.7; KKTs of 3-D grids (7): 16^3 9.7 / 12.5 -> 6.9 /
+  // 7.3, 48^3 22 / 30 -> 17 / 27; QP (4), n = 3300: 9.0 -> 6.9; 64 2-D KKTs
+  // 54 -> 38.  Rows of fewer entries would leave most of eight lanes idle.
+  const int64_t mean = nnz / std::max(n, 1);
+  if (mean >= 96)
+    k_spmv_lanes<64><<<grid_for((int64_t)n * 64, 256), 256, 0, st>>>(n, rp, ci, v, perm_f, iperm_f, x, b, y, nrhs);
+  else if (mean >= 16)
+    k_spmv_lanes<16><<<grid_for((int64_t)n * 16, 256), 256, 0, st>>>(n, rp, ci, v, perm_f, iperm_f, x, b, y, nrhs);
+  else if (mean >= 4)
+    k_spmv_lanes<8><<<grid_for((int64_t)n * 8, 256), 256, 0, st>>>(n, rp, ci, v, perm_f, iperm_f, x, b, y, nrhs);
+  else
+    k_spmv<<<grid_for(n, 256), 256, 0, st>>>(n, rp, ci, v, perm_f, iperm_f, x, b, y, nrhs);
   HIP_LAUNCH_CHECK("spmv");
 }
 

@@ -144,8 +144,8 @@ void launch_fwd_chain(int s, int w, int64_t r, const SnArgs& a, const T* valL, T
 template <typename T>
 void launch_bwd_chain(int s, int w, int64_t r, const SnArgs& a, const T* valL, const T* Z, T* offacc, T* Xf,
                       int nrhs, uint64_t* xb, uint32_t epoch, int* status, hipStream_t st);
-void launch_spmv(int n, const int* rp, const int* ci, const double* v, const int* perm_f, const int* iperm_f,
-                 const double* x, const double* b, double* y, int nrhs, hipStream_t st);
+void launch_spmv(int n, int64_t nnz, const int* rp, const int* ci, const double* v, const int* perm_f,
+                 const int* iperm_f, const double* x, const double* b, double* y, int nrhs, hipStream_t st);
 // GMRES vector work of short vectors in one workgroup (gmres_one: whether
 // n x nrhs is short): after the preconditioned residual z, and after inner
 // step k's preconditioned basis vector in V(k + 1)
