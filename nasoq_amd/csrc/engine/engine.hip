@@ -1514,7 +1514,7 @@ static void gmres_cycle(DeviceFactor& D, const double* b, double* x, int nrhs, i
   auto Vk = [&](int k) { return D.V + (int64_t)k * nn; };
   spmv_ordered(D, x, D.R, nrhs, b);
   apply_solve(D, D.R, D.Xs, nrhs, nullptr, 0);
-  if (gmres_one(n, nrhs) && mr <= MR) {
+  if (gmres_one(n, nrhs)) {
     launch_gmres_begin(n, nrhs, MR, D.gm, D.Xs, D.V, itr, tol_abs, tol_rel, st);
     for (int k = 0; k < mr; ++k) {
       spmv_ordered(D, Vk(k), D.T, nrhs);

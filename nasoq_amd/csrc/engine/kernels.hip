@@ -1729,56 +1729,15 @@ __global__ void k_red_final(const double* part, int nblk, int nv, double* out) {
 }
 // workgroups for a reduction over n rows: enough to cover n, at most cap
 static int red_blocks(int n, int cap) { return (int)std::max<int64_t>(1, std::min<int64_t>(cap, (n + 255) / 256)); }
-// short vectors: one workgroup of 1024 threads, strided per-thread sums and
-// a fixed tree (one launch instead of two; repeated calls agree bit for bit)
-__global__ __launch_bounds__(1024) void k_dot_one(int n, int nrhs, const double* a, const double* b, double* out) {
-  __shared__ double sh[16][MAXRHS];
-  const int t = threadIdx.x, wv = t >> 6, ln = t & 63;
-  double acc[MAXRHS];
-#pragma unroll
-  for (int c = 0; c < MAXRHS; ++c) acc[c] = 0.0;
-  for (int i = t; i < n; i += 1024)
-#pragma unroll
-    for (int c = 0; c < MAXRHS; ++c)
-      if (c < nrhs) acc[c] += a[(int64_t)i * nrhs + c] * b[(int64_t)i * nrhs + c];
-#pragma unroll
-  for (int c = 0; c < MAXRHS; ++c) {
-    if (c >= nrhs) break;
-    const double v = wave_sum(acc[c]);
-    if (ln == 0) sh[wv][c] = v;
-  }
-  __syncthreads();
-  if (t < nrhs) {
-    double s = 0.0;
-    for (int q = 0; q < 16; ++q) s += sh[q][t];
-    out[t] = s;
-  }
-}
-#define DOT_ONE_MAX (1 << 16)  // rows x columns up to which one workgroup takes the dot products
+#define DOT_ONE_MAX (1 << 16)  // rows x columns up to which one workgroup takes an inner step's vector work
 
 void launch_dot(int n, int nrhs, const double* a, const double* b, double* part, int nblk, double* out,
                 hipStream_t st) {
-  if ((int64_t)n * nrhs <= DOT_ONE_MAX) {
-    k_dot_one<<<1, 1024, 0, st>>>(n, nrhs, a, b, out);
-    HIP_LAUNCH_CHECK("dot_one");
-    return;
-  }
   nblk = red_blocks(n, nblk);
   k_dot_partial<<<nblk, 256, 0, st>>>(n, nrhs, a, b, part);
   HIP_LAUNCH_CHECK("dot_partial");
   k_red_final<<<1, 256, 0, st>>>(part, nblk, nrhs, out);
   HIP_LAUNCH_CHECK("dot_final");
-}
-
-// elementwise: r = b - y
-__global__ void k_sub(int64_t count, const double* b, const double* y, double* r) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count;
-       i += (int64_t)gridDim.x * blockDim.x)
-    r[i] = b[i] - y[i];
-}
-void launch_sub(int64_t count, const double* b, const double* y, double* r, hipStream_t st) {
-  k_sub<<<grid_for(count, 256), 256, 0, st>>>(count, b, y, r);
-  HIP_LAUNCH_CHECK("sub");
 }
 
 // y(:,c) = alpha_c * x(:,c) + beta_c * y(:,c) with per-column coefficients
@@ -1944,7 +1903,7 @@ void launch_gmres_scalar(int op, int nrhs, int MR, double* gm, const double* dot
 // took 4 k + 9 launches of about 4 us and 2 us between them, 0.9 ms of the
 // 3 ms that an active-set iteration of the 40 x 40 QP takes with its nine
 // inner steps.  An update and the dot product after it share a pass over the
-// vectors.  The sums are k_dot_one's: strided per-thread sums (thread t has
+// vectors.  The sums are strided per-thread sums (thread t has
 // rows t, t + 1024, ...), then a fixed tree, so repeated calls agree bit for
 // bit.  The columns' state is worked on in LDS (GM_LDS doubles hold it for
 // restart lengths up to 16; beyond, in memory).

@@ -190,7 +190,6 @@ void launch_solve_batch(const int* sysd, int nsys, const int4* info, const int64
 // column), reduced in a fixed order through at most nblk partials
 void launch_dot(int n, int nrhs, const double* a, const double* b, double* part, int nblk, double* out,
                 hipStream_t st);
-void launch_sub(int64_t count, const double* b, const double* y, double* r, hipStream_t st);
 void launch_axpby(int n, int nrhs, const double* coefs, int cstride, const double* x, double* y,
                   const double* mask, int mstride, int mask_off, int mode, hipStream_t st);
 // out = column dots of a and b, then GMRES scalar step op on them (one launch for short vectors)
