@@ -34,9 +34,23 @@ __device__ inline float bf2f(unsigned short h) { return __uint_as_float((unsigne
 __device__ inline float tof(float v) { return v; }
 __device__ inline float tof(unsigned short v) { return bf2f(v); }
 
+enum { EPI_NONE = 0, EPI_RELU = 1, EPI_MASK = 2 };
+// what happens to a product's element (element q of the output, column j) before it is stored
+struct Epilogue {
+  const float* bias = nullptr;  // added when given
+  const float* act = nullptr;   // EPI_MASK: the element is 0 where act is not positive
+  int op = EPI_NONE;
+  __device__ float apply(float v, int64_t q, int j) const {
+    if (bias) v += bias[j];
+    if (op == EPI_RELU && v < 0.f) v = 0.f;
+    if (op == EPI_MASK && !(act[q] > 0.f)) v = 0.f;
+    return v;
+  }
+};
+
 #define GT 64   // output tile
 #define GKC 32  // k chunk staged in LDS
-// C(i, j) = alpha sum_k a(i, k) b(k, j) + beta C(i, j), a(i, k) = A[i sa0 + k sa1],
+// C(i, j) = f(sum_k a(i, k) b(k, j)), a(i, k) = A[i sa0 + k sa1],
 // b(k, j) = B[k sb0 + j sb1]; operands rounded to BF16, FP32 accumulation.
 // A wave owns a 32 x 32 quadrant = 2 x 2 MFMA blocks of 16 x 16: operand lane l
 // holds row (or column) l % 16 and k = 4 (l / 16) .. + 3, accumulator element e
@@ -44,7 +58,7 @@ __device__ inline float tof(unsigned short v) { return bf2f(v); }
 template <typename TA, typename TB>
 __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, const TA* A, int64_t sa0, int64_t sa1,
                                                    const TB* B, int64_t sb0, int64_t sb1, float* C, int ldc,
-                                                   float alpha, float beta) {
+                                                   Epilogue f) {
   __shared__ unsigned short As[GT][GKC + 4];  // [row][k]
   __shared__ unsigned short Bs[GT][GKC + 4];  // [column][k]
   const int t = threadIdx.x, wv = t >> 6, ln = t & 63;
@@ -95,47 +109,47 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, const TA
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = i0 + wr + 16 * r + 4 * (ln >> 4) + e, j = j0 + wc + 16 * c + (ln & 15);
-        if (i < M && j < N) {
-          float* p = C + (int64_t)i * ldc + j;
-          *p = alpha * acc[r][c][e] + (beta != 0.f ? beta * *p : 0.f);
-        }
+        if (i < M && j < N) C[(int64_t)i * ldc + j] = f.apply(acc[r][c][e], (int64_t)i * ldc + j, j);
       }
 }
 template <typename TA, typename TB>
 static void gemm(int M, int N, int K, const TA* A, int64_t sa0, int64_t sa1, const TB* B, int64_t sb0, int64_t sb1,
-                 float* C, int ldc, hipStream_t st) {
+                 float* C, int ldc, hipStream_t st, const Epilogue& f = {}) {
   dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT);
-  k_gemm_bf16<TA, TB><<<grid, 256, 0, st>>>(M, N, K, A, sa0, sa1, B, sb0, sb1, C, ldc, 1.f, 0.f);
+  k_gemm_bf16<TA, TB><<<grid, 256, 0, st>>>(M, N, K, A, sa0, sa1, B, sb0, sb1, C, ldc, f);
   HIP_LAUNCH_CHECK("gemm_bf16");
 }
 
 // --------------------------------------------------------------------------
 // The products with a weight matrix: C(i, j) = f(sum_k A(i, k) W(k, j)), A
 // FP32 with k contiguous (rounded to BF16 as it is read), W the BF16 copy,
-// W(k, j) = W[k sw0 + j sw1] with one of the strides 1.  A minibatch has few
-// rows, so 64 x 64 tiles gave 16 workgroups on 256 CUs and a chain of K / 32
-// staged chunks, 62 us at 64 x 1024 x 1024.  Here a workgroup has a 32 x 32
-// tile (64 workgroups there), its four waves take every fourth 16-deep slice
-// of k with operands loaded lane by lane, several slices in flight, and meet
-// in LDS in a fixed order: 11 us.  f: bias (added when given), ReLU, or the
-// mask dA(i, j) = 0 where act(i, j) <= 0 of the backward pass, so that no
-// separate pass follows.
+// W(k, j) = W[k sw0 + j sw1] with one of the strides 1.  f: bias (added when
+// given), ReLU, or the mask dA(i, j) = 0 where act(i, j) <= 0 of the backward
+// pass, so that no separate pass follows.
+//
+// Every element is summed by one accumulator over ascending 16-deep slices
+// of k, here as in k_gemm_bf16, so both kernels give the same bits.  That
+// order is kept on purpose: an activation on a BF16 rounding boundary goes to
+// the other side when its sum is taken in another order, and Adam turns a
+// gradient of rounding size into a step of a whole learning rate.
+//
+// A minibatch has few rows: 64 x 64 tiles give 16 workgroups on 256 CUs and a
+// chain of K / 32 staged chunks, 64 to 73 us at 64 x 1024 x 1024.  The chain
+// of MFMAs itself is short (K / 16 of them), the loads are what it waits for,
+// so one wave takes one 16 x 16 tile, reads its operands lane by lane without
+// LDS and has WU to 2 WU slices in flight: 10.8 us with k contiguous in W,
+// 20.1 us with j contiguous.  Eight or sixteen slices, or four waves a
+// workgroup, were no faster there (10.5 to 18 us).
 // --------------------------------------------------------------------------
-enum { EPI_NONE = 0, EPI_RELU = 1, EPI_MASK = 2 };
-constexpr int WT = 32;  // output tile
+constexpr int WU = 4;  // slices loaded together
 // four consecutive k of A's row, zero beyond K
 template <bool VEC>
-__device__ inline s4 load_a(const float* row, int k, int K) {
-  float v[4];
-  if (VEC) {  // K and the rows are multiples of four
-    const f4 x = k < K ? *reinterpret_cast<const f4*>(row + k) : f4{0.f, 0.f, 0.f, 0.f};
-    for (int e = 0; e < 4; ++e) v[e] = x[e];
-  } else {
-    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? row[k + e] : 0.f;
-  }
-  s4 r;
-  for (int e = 0; e < 4; ++e) r[e] = (short)f2bf(v[e]);
-  return r;
+__device__ inline f4 load_a(const float* row, int k, int K) {
+  if (VEC)  // K and the rows are multiples of four
+    return k < K ? *reinterpret_cast<const f4*>(row + k) : f4{0.f, 0.f, 0.f, 0.f};
+  f4 v;
+  for (int e = 0; e < 4; ++e) v[e] = k + e < K ? row[k + e] : 0.f;
+  return v;
 }
 template <bool VEC>
 __device__ inline s4 load_w(const unsigned short* col, int64_t sw0, int k, int K) {
@@ -145,71 +159,66 @@ __device__ inline s4 load_w(const unsigned short* col, int64_t sw0, int k, int K
   return r;
 }
 template <bool VEC>
-__global__ __launch_bounds__(256) void k_gemm_weight(int M, int N, int K, const float* A, int lda,
-                                                     const unsigned short* W, int64_t sw0, int64_t sw1, float* C,
-                                                     int ldc, const float* bias, const float* act, int epi) {
-  __shared__ float red[4][WT][WT + 1];
-  const int t = threadIdx.x, wv = t >> 6, ln = t & 63, li = ln & 15, lk = 4 * (ln >> 4);
-  const int i0 = blockIdx.y * WT, j0 = blockIdx.x * WT;
+__global__ __launch_bounds__(64) void k_gemm_weight(int M, int N, int K, const float* A, int lda,
+                                                    const unsigned short* W, int64_t sw0, int64_t sw1, float* C,
+                                                    int ldc, Epilogue f) {
+  const int ln = threadIdx.x, li = ln & 15, lk = 4 * (ln >> 4);
+  const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16;
   // rows and columns beyond the matrix read the last one and are not stored
-  const float* ar[2];
-  const unsigned short* wc[2];
+  const float* ar = A + (int64_t)min(i0 + li, M - 1) * lda;
+  const unsigned short* wc = W + (int64_t)min(j0 + li, N - 1) * sw1;
+  f4 acc = {0.f, 0.f, 0.f, 0.f}, a[WU];
+  s4 b[WU];
+  auto fetch = [&](int k0) {
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    ar[r] = A + (int64_t)min(i0 + 16 * r + li, M - 1) * lda;
-    wc[r] = W + (int64_t)min(j0 + 16 * r + li, N - 1) * sw1;
-  }
-  f4 acc[2][2];
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int c = 0; c < 2; ++c) acc[r][c] = f4{0.f, 0.f, 0.f, 0.f};
-  constexpr int U = 4;  // slices in flight
-  for (int k0 = 16 * wv; k0 < K; k0 += 64 * U) {
-    s4 a[U][2], b[U][2];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        a[u][r] = load_a<VEC>(ar[r], k0 + 64 * u + lk, K);
-        b[u][r] = load_w<VEC>(wc[r], sw0, k0 + 64 * u + lk, K);
-      }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[u][r], b[u][c], acc[r][c], 0, 0, 0);
-  }
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) red[wv][16 * r + lk + e][16 * c + li] = acc[r][c][e];
-  __syncthreads();
-  for (int q = t; q < WT * WT; q += 256) {
-    const int i = q / WT, j = q % WT;
-    if (i0 + i < M && j0 + j < N) {
-      float v = (red[0][i][j] + red[1][i][j]) + (red[2][i][j] + red[3][i][j]);
-      if (bias) v += bias[j0 + j];
-      if (epi == EPI_RELU && v < 0.f) v = 0.f;
-      if (epi == EPI_MASK && !(act[(int64_t)(i0 + i) * ldc + j0 + j] > 0.f)) v = 0.f;
-      C[(int64_t)(i0 + i) * ldc + j0 + j] = v;
+    for (int u = 0; u < WU; ++u) {
+      a[u] = load_a<VEC>(ar, k0 + 16 * u + lk, K);
+      b[u] = load_w<VEC>(wc, sw0, k0 + 16 * u + lk, K);
     }
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < K; k0 += 16 * WU) {
+    f4 x[WU];
+    s4 y[WU];
+#pragma unroll
+    for (int u = 0; u < WU; ++u) {
+      x[u] = a[u];
+      y[u] = b[u];
+    }
+    fetch(k0 + 16 * WU);  // the next slices' loads beside these slices' MFMAs (zeros beyond K)
+#pragma unroll
+    for (int u = 0; u < WU; ++u) {
+      s4 xa;
+      for (int e = 0; e < 4; ++e) xa[e] = (short)f2bf(x[u][e]);
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xa, y[u], acc, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int i = i0 + lk + e, j = j0 + li;
+    if (i < M && j < N) C[(int64_t)i * ldc + j] = f.apply(acc[e], (int64_t)i * ldc + j, j);
   }
 }
 static void gemm_weight(int M, int N, int K, const float* A, const unsigned short* W, int64_t sw0, int64_t sw1,
-                        float* C, const float* bias, const float* act, int epi, hipStream_t st) {
-  const dim3 grid((N + WT - 1) / WT, (M + WT - 1) / WT);
+                        float* C, const Epilogue& f, hipStream_t st) {
+  // Many rows fill the chip with 64 x 64 tiles too, which read each operand a
+  // quarter as often.  64 x 64 tiles / one wave a tile, us, K = 1024, N = 1024:
+  // k contiguous in W, M = 64: 73 / 10.8, 1024: 80 / 60, 2048: 132 / 116,
+  // 4096: 233 / 226; j contiguous (two-byte loads), M = 64: 64 / 20,
+  // 1024: 100 / 45, 2048: 101 / 87, 4096: 155 / 168; 1024 x 4000: 154 / 172.
+  // (The 16-row tiles also end at the grid's 65,535 rows of workgroups.)
+  if ((sw0 != 1 && (int64_t)M * N > (int64_t)1 << 21) || M > 65535 * 16) {
+    gemm(M, N, K, A, K, 1, W, sw0, sw1, C, N, st, f);
+    return;
+  }
+  const dim3 grid((N + 15) / 16, (M + 15) / 16);
   // four-element loads: rows of A (and of W, read along k) on their alignment
   const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                    (sw0 != 1 || (sw1 % 4 == 0 && reinterpret_cast<uintptr_t>(W) % 8 == 0));
   if (vec)
-    k_gemm_weight<true><<<grid, 256, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, bias, act, epi);
+    k_gemm_weight<true><<<grid, 64, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, f);
   else
-    k_gemm_weight<false><<<grid, 256, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, bias, act, epi);
+    k_gemm_weight<false><<<grid, 64, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, f);
   HIP_LAUNCH_CHECK("gemm_weight");
 }
 
@@ -234,22 +243,25 @@ __global__ void k_sigmoid(const float* Z, float* P, int64_t n) {
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x)
     P[q] = 1.f / (1.f + expf(-Z[q]));
 }
-// db(j) = sum_b dZ(b, j): 64 columns a workgroup, its four waves take every
-// fourth row, a fixed order
-__global__ __launch_bounds__(256) void k_colsum(const float* dZ, int rows, int cols, float* db) {
-  __shared__ float sh[4][64];
-  const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63, j = blockIdx.x * 64 + ln;
+// db(j) = sum_b dZ(b, j), one thread per column in ascending rows (the order
+// is kept for the reason given at k_gemm_weight); sixteen rows' loads together
+constexpr int CSU = 16;
+__global__ __launch_bounds__(64) void k_colsum(const float* dZ, int rows, int cols, float* db) {
+  const int j = blockIdx.x * 64 + threadIdx.x;
+  if (j >= cols) return;
   float s = 0.f;
-  if (j < cols) {
-#pragma unroll 8
-    for (int b = wv; b < rows; b += 4) s += dZ[(int64_t)b * cols + j];
+  for (int b0 = 0; b0 < rows; b0 += CSU) {
+    float v[CSU];
+#pragma unroll
+    for (int u = 0; u < CSU; ++u) v[u] = b0 + u < rows ? dZ[(int64_t)(b0 + u) * cols + j] : 0.f;
+#pragma unroll
+    for (int u = 0; u < CSU; ++u)
+      if (b0 + u < rows) s += v[u];
   }
-  sh[wv][ln] = s;
-  __syncthreads();
-  if (wv == 0 && j < cols) db[j] = (sh[0][ln] + sh[1][ln]) + (sh[2][ln] + sh[3][ln]);
+  db[j] = s;
 }
 static void colsum(const float* dZ, int rows, int cols, float* db, hipStream_t st) {
-  k_colsum<<<(cols + 63) / 64, 256, 0, st>>>(dZ, rows, cols, db);
+  k_colsum<<<(cols + 63) / 64, 64, 0, st>>>(dZ, rows, cols, db);
 }
 // Adam (Kingma & Ba 2015) on the FP32 master parameters, then their BF16 copy
 __global__ void k_adam(float* P, unsigned short* Pb, const float* G, float* Mo, float* Vo, int64_t n, float lr,
@@ -315,9 +327,9 @@ struct Mlp {
     if (st) (void)hipStreamDestroy(st);
   }
   void forward(int B) {
-    gemm_weight(B, h1, in, X, Pb + oW1, 1, in, A1, P + ob1, nullptr, EPI_RELU, st);
-    gemm_weight(B, h2, h1, A1, Pb + oW2, 1, h1, A2, P + ob2, nullptr, EPI_RELU, st);
-    gemm_weight(B, out, h2, A2, Pb + oW3, 1, h2, Z3, P + ob3, nullptr, EPI_NONE, st);
+    gemm_weight(B, h1, in, X, Pb + oW1, 1, in, A1, {P + ob1, nullptr, EPI_RELU}, st);
+    gemm_weight(B, h2, h1, A1, Pb + oW2, 1, h1, A2, {P + ob2, nullptr, EPI_RELU}, st);
+    gemm_weight(B, out, h2, A2, Pb + oW3, 1, h2, Z3, {P + ob3, nullptr, EPI_NONE}, st);
     HIP_LAUNCH_CHECK("mlp forward");
   }
   // gradients of the mean BCE over the batch into G; loss into *loss (device)
@@ -327,10 +339,10 @@ struct Mlp {
     k_bce<<<ew_grid(no), 256, 0, st>>>(Z3, Y, no, dZ3, loss);
     gemm(out, h2, B, dZ3, 1, out, A2, h2, 1, G + oW3, h2, st);  // dW3 = dZ3^T A2
     colsum(dZ3, B, out, G + ob3, st);
-    gemm_weight(B, h2, out, dZ3, Pb + oW3, h2, 1, dA2, nullptr, A2, EPI_MASK, st);  // dA2 = dZ3 W3 where A2 > 0
+    gemm_weight(B, h2, out, dZ3, Pb + oW3, h2, 1, dA2, {nullptr, A2, EPI_MASK}, st);  // dA2 = dZ3 W3 where A2 > 0
     gemm(h2, h1, B, dA2, 1, h2, A1, h1, 1, G + oW2, h1, st);  // dW2 = dA2^T A1
     colsum(dA2, B, h2, G + ob2, st);
-    gemm_weight(B, h1, h2, dA2, Pb + oW2, h1, 1, dA1, nullptr, A1, EPI_MASK, st);  // dA1 = dA2 W2 where A1 > 0
+    gemm_weight(B, h1, h2, dA2, Pb + oW2, h1, 1, dA1, {nullptr, A1, EPI_MASK}, st);  // dA1 = dA2 W2 where A1 > 0
     gemm(h1, in, B, dA1, 1, h1, X, in, 1, G + oW1, in, st);  // dW1 = dA1^T X
     colsum(dA1, B, h1, G + ob1, st);
     HIP_LAUNCH_CHECK("mlp backward");
