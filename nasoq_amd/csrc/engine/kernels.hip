@@ -1729,7 +1729,6 @@ __global__ void k_red_final(const double* part, int nblk, int nv, double* out) {
 }
 // workgroups for a reduction over n rows: enough to cover n, at most cap
 static int red_blocks(int n, int cap) { return (int)std::max<int64_t>(1, std::min<int64_t>(cap, (n + 255) / 256)); }
-#define DOT_ONE_MAX (1 << 16)  // rows x columns up to which one workgroup takes an inner step's vector work
 
 void launch_dot(int n, int nrhs, const double* a, const double* b, double* part, int nblk, double* out,
                 hipStream_t st) {
@@ -1897,7 +1896,7 @@ void launch_gmres_scalar(int op, int nrhs, int MR, double* gm, const double* dot
 
 // --------------------------------------------------------------------------
 // The vector work of GMRES on short vectors (rows x columns up to
-// DOT_ONE_MAX) in one workgroup: k_gmres_begin after the preconditioned
+// GMRES_ONE_MAX) in one workgroup: k_gmres_begin after the preconditioned
 // residual, k_gmres_step after each preconditioned basis vector.  Launch by
 // launch (a dot product with its scalar step, an update, ...) an inner step
 // took 4 k + 9 launches of about 4 us and 2 us between them, 0.9 ms of the
@@ -2090,7 +2089,15 @@ __global__ __launch_bounds__(1024) void k_gmres_step(int n, int MR, int mr, int 
   }
   gm_close<NR>(G, gm, MR);
 }
-bool gmres_one(int n, int nrhs) { return (int64_t)n * nrhs <= DOT_ONE_MAX; }
+// Rows x columns up to which one workgroup takes an inner step: its passes run
+// on one CU, so their time grows with the vectors, while the launches' does
+// not.  One cycle's vector work in a captured graph, one workgroup / launches,
+// us: GMRES(2), 1 column, 8192 rows: 59 / 107, 16384: 91 / 106, 24576:
+// 122 / 108, 65536: 277 / 106; 8 columns x 2048 rows: 200 / 214, x 3072:
+// 269 / 215, x 8192: 617 / 218; GMRES(3), 1 x 16384: 165 / 172, 8 x 2048:
+// 400 / 365; GMRES(8), 1 x 12288: 627 / 718, 1 x 16384: 790 / 724.
+constexpr int64_t GMRES_ONE_MAX = 1 << 14;
+bool gmres_one(int n, int nrhs) { return (int64_t)n * nrhs <= GMRES_ONE_MAX; }
 void launch_gmres_begin(int n, int nrhs, int MR, double* gm, const double* z, double* V, int itr, double tol_abs,
                         double tol_rel, hipStream_t st) {
   auto go = [&](auto nr) {

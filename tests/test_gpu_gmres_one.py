@@ -54,3 +54,28 @@ def test_refinement_matches_dense_gmres(nrhs, mr, cycles):
         bound = 1e-3 * np.linalg.norm(ref - X0[:, c]) + 1e-13 * np.linalg.norm(ref)
         assert np.linalg.norm(X[:, c] - ref) <= bound, c
     s.close()
+
+
+@pytest.mark.parametrize("target", [0.0, 1e-13])
+def test_columns_agree_across_the_limit(target):
+    # 4352 rows: three columns' steps take one workgroup, four columns' take
+    # launches; every column is its own iteration, so each agrees with the
+    # column solved alone
+    n, Ap, Ai, Ax, B = P.kkt_config(16, 256, 8, seed=3, nrhs=4)
+    assert 3 * n <= 1 << 14 < 4 * n
+    s = lbl.SolverSettings(n, Ap, Ai, Ax)
+    s.reg_diag, s.precision, s.target_bwd_err = 1e-9, lbl.F32, target
+    s.max_inner_iter, s.req_ref_iter = 3, 2
+    assert s.symbolic_analysis() == 1
+    s.numerical_factorization()
+    for nrhs in (3, 4):
+        print(f"case gmres limit nrhs={nrhs} target={target}", flush=True)
+        X = s.solve_only(B[:, :nrhs])
+        for c in range(nrhs):
+            x = s.solve_only(B[:, c])
+            # backward errors of at most 1e-13 each and a condition number of
+            # 400 (1-norm): a forward difference of at most 8e-11, in the
+            # 2-norm with a margin of ten
+            assert np.linalg.norm(X[:, c] - x) <= 1e-9 * np.linalg.norm(x), c
+            assert s.backward_error(B[:, c], X[:, c]) <= 1e-13, c
+    s.close()
