@@ -8,10 +8,9 @@
 // Engine extension: the reference factors one KKT per SolverSettings.
 #include <cmath>
 #include <cstring>
-#include <new>
-#include <stdexcept>
 #include <vector>
 
+#include "capi_guard.hpp"
 #include "engine/handle.hpp"
 #include "lblg.h"
 
@@ -41,7 +40,7 @@ extern "C" int lblg_batch_create(lblg_handle** out, int count, const int* n, con
     nnz += Ap[k][n[k]];
   }
   if (N > 0x7fffffff || nnz > 0x7fffffff) return LBLG_ERR_ARG;  // the CSC index type is int
-  try {
+  return lblg::guarded([&] {
     std::vector<int> P(N + 1), I(nnz);
     std::vector<double> X(nnz);
     std::vector<int64_t> off(count + 1, 0);
@@ -64,15 +63,13 @@ extern "C" int lblg_batch_create(lblg_handle** out, int count, const int* n, con
     if (rc != LBLG_OK) return rc;
     reinterpret_cast<Handle*>(*out)->batch_off = std::move(off);
     return LBLG_OK;
-  } catch (const std::bad_alloc&) {
-    return LBLG_ERR_NOMEM;
-  }
+  });
 }
 
 extern "C" int lblg_batch_analyze(lblg_handle* hh, const lblg_settings* s) {
   Handle* h = reinterpret_cast<Handle*>(hh);
   if (!h || !s || h->batch_off.size() < 2) return LBLG_ERR_ARG;
-  try {
+  return lblg::guarded([&] {
     const int count = (int)h->batch_off.size() - 1;
     std::vector<int> perm(h->n);
     std::vector<int> bp, bi, order;
@@ -94,9 +91,7 @@ extern "C" int lblg_batch_analyze(lblg_handle* hh, const lblg_settings* s) {
     lblg_settings st = *s;
     st.ordering = LBLG_ORDER_GIVEN;
     return lblg_analyze(hh, &st, perm.data(), nullptr);
-  } catch (const std::bad_alloc&) {
-    return LBLG_ERR_NOMEM;
-  }
+  });
 }
 
 extern "C" int lblg_batch_info(const lblg_handle* hh, int* count, int64_t* offsets) {
@@ -115,7 +110,7 @@ extern "C" int lblg_batch_backward_errors(const lblg_handle* hh, int nrhs, const
   const Handle* h = reinterpret_cast<const Handle*>(hh);
   if (!h || !B || !X || !err || nrhs < 1 || ldb < h->n || ldx < h->n || h->batch_off.size() < 2)
     return LBLG_ERR_ARG;
-  try {
+  return lblg::guarded([&] {
     const int count = (int)h->batch_off.size() - 1;
     const double reg = h->set.regularization == 1 ? h->set.reg_diag : -1.0;
     auto val = [&](int q, int j) { return (h->Ai[q] == j && std::fabs(h->Ax[q]) < reg) ? 0.0 : h->Ax[q]; };
@@ -150,7 +145,5 @@ extern "C" int lblg_batch_backward_errors(const lblg_handle* hh, int nrhs, const
       }
     }
     return LBLG_OK;
-  } catch (const std::bad_alloc&) {
-    return LBLG_ERR_NOMEM;
-  }
+  });
 }

@@ -3,50 +3,31 @@
 // interface each function replaces.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
-#include <new>
 #include <stdexcept>
 #include <vector>
 
+#include "capi_guard.hpp"
 #include "engine/device.hpp"
 #include "engine/engine.hpp"
 #include "engine/handle.hpp"
 #include "engine/kernels.hpp"
 #include "lblg.h"
 
+using lblg::guarded;
 using lblg::Handle;
 
-namespace {
-thread_local char g_last_error[512] = {0};
-void set_error(const char* what) {
+static thread_local char g_last_error[512] = {0};
+
+namespace lblg {
+void set_last_error(const char* what) {
   std::strncpy(g_last_error, what, sizeof(g_last_error) - 1);
   g_last_error[sizeof(g_last_error) - 1] = 0;
 }
-}  // namespace
-
-namespace lblg {
-void set_last_error(const char* what) { set_error(what); }
 }  // namespace lblg
-
-namespace {
-template <typename F>
-int guarded(F f) {
-  try {
-    return f();
-  } catch (const std::bad_alloc&) {
-    set_error("allocation failed");
-    return LBLG_ERR_NOMEM;
-  } catch (const std::invalid_argument& e) {
-    set_error(e.what());
-    return LBLG_ERR_ARG;
-  } catch (const std::exception& e) {
-    set_error(e.what());
-    return LBLG_ERR_DEVICE;
-  }
-}
-}  // namespace
 
 extern "C" const char* lblg_last_error(void) { return g_last_error; }
 
@@ -97,17 +78,23 @@ extern "C" int lblg_update_values(lblg_handle* hh, int64_t count, const int64_t*
   const int64_t nnz = (int64_t)h->Ax.size();
   for (int64_t k = 0; k < count; ++k)
     if (idx[k] < 0 || idx[k] >= nnz) return LBLG_ERR_ARG;
-  if (h->changed_flag.size() != h->Ax.size()) h->changed_flag.assign(h->Ax.size(), 0);
-  for (int64_t k = 0; k < count; ++k) {
-    const int64_t q = idx[k];
-    h->Ax[q] = vals[k];
-    if (!h->changed_flag[q]) {
-      h->changed_flag[q] = 1;
-      h->changed.push_back(q);
+  return guarded([&] {
+    if (h->changed_flag.size() != h->Ax.size()) h->changed_flag.assign(h->Ax.size(), 0);
+    int64_t fresh = 0;  // entries new to the list: its room first, so that a failure changes no value
+    for (int64_t k = 0; k < count; ++k) fresh += !h->changed_flag[idx[k]];
+    if (h->changed.size() + fresh > h->changed.capacity())
+      h->changed.reserve(std::max(h->changed.size() + fresh, 2 * h->changed.capacity()));
+    for (int64_t k = 0; k < count; ++k) {
+      const int64_t q = idx[k];
+      h->Ax[q] = vals[k];
+      if (!h->changed_flag[q]) {
+        h->changed_flag[q] = 1;
+        h->changed.push_back(q);
+      }
     }
-  }
-  if (count > 0) h->factored = false;
-  return LBLG_OK;
+    if (count > 0) h->factored = false;
+    return LBLG_OK;
+  });
 }
 
 extern "C" int64_t lblg_refactored_supernodes(const lblg_handle* hh) {
@@ -258,8 +245,11 @@ extern "C" int lblg_inertia(lblg_handle* hh, int64_t* pos, int64_t* neg, int64_t
   Handle* h = reinterpret_cast<Handle*>(hh);
   if (!h || !pos || !neg || !zero) return LBLG_ERR_ARG;
   if (!h->factored) return LBLG_ERR_STATE;
-  std::vector<double> d(2 * (size_t)h->n);
-  int rc = lblg_get_factor(hh, nullptr, d.data(), nullptr, nullptr);
+  std::vector<double> d;
+  int rc = guarded([&] {
+    d.resize(2 * (size_t)h->n);
+    return lblg_get_factor(hh, nullptr, d.data(), nullptr, nullptr);
+  });
   if (rc) return rc;
   const int n = h->n;
   int64_t a = 0, b = 0, z = 0;
@@ -339,37 +329,43 @@ extern "C" int lblg_selftest_mfma(const double* A, const double* B, double* C, i
 extern "C" int lblg_set_kernel_timing(lblg_handle* hh, int on) {
   Handle* h = reinterpret_cast<Handle*>(hh);
   if (!h || !h->dev) return LBLG_ERR_STATE;
-  h->dev->resolve_timing();
-  h->dev->timing = on != 0;
-  h->dev->timing_only.clear();
-  if (on) h->dev->ktime.clear();
-  return LBLG_OK;
+  return guarded([&] {
+    h->dev->resolve_timing();
+    h->dev->timing = on != 0;
+    h->dev->timing_only.clear();
+    if (on) h->dev->ktime.clear();
+    return LBLG_OK;
+  });
 }
 
 extern "C" int lblg_set_kernel_timing_only(lblg_handle* hh, const char* name) {
   Handle* h = reinterpret_cast<Handle*>(hh);
   if (!h || !h->dev) return LBLG_ERR_STATE;
   if (!name || !*name) return LBLG_ERR_ARG;
-  h->dev->resolve_timing();
-  h->dev->timing_only.clear();
-  for (const char* p = name; *p;) {  // comma-separated family names
-    const char* e = p;
-    while (*e && *e != ',') ++e;
-    if (e > p) h->dev->timing_only.insert(std::string(p, e));
-    p = *e ? e + 1 : e;
-  }
-  if (h->dev->timing_only.empty()) return LBLG_ERR_ARG;
-  h->dev->timing = true;
-  h->dev->ktime.clear();
-  return LBLG_OK;
+  return guarded([&] {
+    h->dev->resolve_timing();
+    h->dev->timing_only.clear();
+    for (const char* p = name; *p;) {  // comma-separated family names
+      const char* e = p;
+      while (*e && *e != ',') ++e;
+      if (e > p) h->dev->timing_only.insert(std::string(p, e));
+      p = *e ? e + 1 : e;
+    }
+    if (h->dev->timing_only.empty()) return LBLG_ERR_ARG;
+    h->dev->timing = true;
+    h->dev->ktime.clear();
+    return LBLG_OK;
+  });
 }
 
 extern "C" int lblg_kernel_time(lblg_handle* hh, const char* name, double* total_ms, int64_t* launches) {
   Handle* h = reinterpret_cast<Handle*>(hh);
   if (!h || !h->dev || !name) return LBLG_ERR_ARG;
-  h->dev->resolve_timing();
-  auto it = h->dev->ktime.find(name);
-  if (total_ms) *total_ms = it == h->dev->ktime.end() ? 0.0 : it->second.first;
-  if (launches) *launches = it == h->dev->ktime.end() ? 0 : it->second.second;
-  return LBLG_OK;
+  return guarded([&] {
+    h->dev->resolve_timing();
+    auto it = h->dev->ktime.find(name);
+    if (total_ms) *total_ms = it == h->dev->ktime.end() ? 0.0 : it->second.first;
+    if (launches) *launches = it == h->dev->ktime.end() ? 0 : it->second.second;
+    return LBLG_OK;
+  });
 }

@@ -1,33 +1,16 @@
 // C-ABI of the NASOQ QP solver (include/lblg.h, lblg_qp_*).
 #include <cstring>
-#include <new>
+#include <memory>
 #include <stdexcept>
 
+#include "capi_guard.hpp"
 #include "host/qp.hpp"
 #include "lblg.h"
 
+using lblg::guarded;
 using lblg::QpSolver;
 
-namespace lblg {
-void set_last_error(const char* what);  // capi_numeric.cpp (lblg_last_error)
-}
-
 namespace {
-template <typename F>
-int guarded(F f) {
-  try {
-    return f();
-  } catch (const std::bad_alloc&) {
-    lblg::set_last_error("allocation failed");
-    return LBLG_ERR_NOMEM;
-  } catch (const std::invalid_argument& e) {
-    lblg::set_last_error(e.what());
-    return LBLG_ERR_ARG;
-  } catch (const std::exception& e) {
-    lblg::set_last_error(e.what());
-    return LBLG_ERR_DEVICE;
-  }
-}
 bool valid_csc(int nrow, int ncol, const int* p, const int* i) {
   if (!p || (p[ncol] > 0 && !i) || p[0] != 0) return false;
   for (int j = 0; j < ncol; ++j) {
@@ -72,7 +55,7 @@ extern "C" int lblg_qp_create(lblg_qp** out, int n, const int* Hp, const int* Hi
   if (me > 0 && (!valid_csc(me, n, Ap, Ai) || !Ax || !a)) return LBLG_ERR_ARG;
   if (mi > 0 && (!valid_csc(mi, n, Bp, Bi) || !Bx || !b)) return LBLG_ERR_ARG;
   return guarded([&] {
-    QpSolver* s = new QpSolver();
+    std::unique_ptr<QpSolver> s(new QpSolver());
     s->n = n;
     s->me = me;
     s->mi = mi;
@@ -97,7 +80,7 @@ extern "C" int lblg_qp_create(lblg_qp** out, int n, const int* Hp, const int* Hi
     s->primal.assign(n, 0.0);
     s->dual.assign(mi, 0.0);
     s->dual_eq.assign(me, 0.0);
-    *out = reinterpret_cast<lblg_qp*>(s);
+    *out = reinterpret_cast<lblg_qp*>(s.release());
     return LBLG_OK;
   });
 }
@@ -132,10 +115,12 @@ extern "C" int lblg_qp_set_settings(lblg_qp* qp, const lblg_qp_settings* st) {
 extern "C" int lblg_qp_set_linear(lblg_qp* qp, const double* q, const double* a, const double* b) {
   QpSolver* s = reinterpret_cast<QpSolver*>(qp);
   if (!s) return LBLG_ERR_ARG;
-  if (q) s->q.assign(q, q + s->n);
-  if (a && s->me) s->a.assign(a, a + s->me);
-  if (b && s->mi) s->b.assign(b, b + s->mi);
-  return LBLG_OK;
+  return guarded([&] {
+    if (q) s->q.assign(q, q + s->n);
+    if (a && s->me) s->a.assign(a, a + s->me);
+    if (b && s->mi) s->b.assign(b, b + s->mi);
+    return LBLG_OK;
+  });
 }
 
 extern "C" int lblg_qp_analyze(lblg_qp* qp) {
@@ -271,13 +256,15 @@ extern "C" int lblg_kkt_edit(lblg_qp* qp, int add, int count, const int* rows) {
   if (!s->analysed) return LBLG_ERR_STATE;
   for (int k = 0; k < count; ++k)
     if (rows[k] < 0 || rows[k] >= s->mi) return LBLG_ERR_ARG;
-  for (int k = 0; k < count; ++k) {
-    const int c = rows[k];
-    s->edit_kkt(add != 0, c);
-    if (add && !s->used[c]) s->update_active_set(true, c);
-    else if (!add && s->used[c]) s->update_active_set(false, c);
-  }
-  return LBLG_OK;
+  return guarded([&] {
+    for (int k = 0; k < count; ++k) {
+      const int c = rows[k];
+      s->edit_kkt(add != 0, c);
+      if (add && !s->used[c]) s->update_active_set(true, c);
+      else if (!add && s->used[c]) s->update_active_set(false, c);
+    }
+    return LBLG_OK;
+  });
 }
 
 extern "C" int lblg_kkt_factor(lblg_qp* qp) {

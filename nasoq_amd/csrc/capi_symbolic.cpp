@@ -2,9 +2,9 @@
 // symbolic analysis.  See include/lblg.h for the reference interface each
 // function replaces.
 #include <cstring>
-#include <new>
-#include <stdexcept>
+#include <memory>
 
+#include "capi_guard.hpp"
 #include "engine/device.hpp"
 #include "engine/handle.hpp"
 #include "lblg.h"
@@ -51,18 +51,16 @@ extern "C" int lblg_create(lblg_handle** out, int n, const int* Ap, const int* A
   if (!out) return LBLG_ERR_ARG;
   *out = nullptr;
   if (!valid_lower_csc(n, Ap, Ai) || !Ax) return LBLG_ERR_ARG;
-  try {
-    Handle* h = new Handle;
+  return lblg::guarded([&] {
+    std::unique_ptr<Handle> h(new Handle);
     h->n = n;
     h->Ap.assign(Ap, Ap + n + 1);
     h->Ai.assign(Ai, Ai + Ap[n]);
     h->Ax.assign(Ax, Ax + Ap[n]);
     lblg_default_settings(&h->set);
-    *out = reinterpret_cast<lblg_handle*>(h);
+    *out = reinterpret_cast<lblg_handle*>(h.release());
     return LBLG_OK;
-  } catch (const std::bad_alloc&) {
-    return LBLG_ERR_NOMEM;
-  }
+  });
 }
 
 extern "C" int lblg_destroy(lblg_handle* hh) {
@@ -72,14 +70,12 @@ extern "C" int lblg_destroy(lblg_handle* hh) {
 
 extern "C" int lblg_order_nd(int n, const int* Ap, const int* Ai, int* perm) {
   if (!valid_lower_csc(n, Ap, Ai) || !perm) return LBLG_ERR_ARG;
-  try {
+  return lblg::guarded([&] {
     std::vector<int> p;
     lblg::nested_dissection(lblg::CscView{n, Ap, Ai}, p);
     std::memcpy(perm, p.data(), sizeof(int) * n);
     return LBLG_OK;
-  } catch (const std::bad_alloc&) {
-    return LBLG_ERR_NOMEM;
-  }
+  });
 }
 
 extern "C" int lblg_analyze(lblg_handle* hh, const lblg_settings* s, const int* perm, const int* extra) {
@@ -87,7 +83,7 @@ extern "C" int lblg_analyze(lblg_handle* hh, const lblg_settings* s, const int* 
   if (!h || !s) return LBLG_ERR_ARG;
   if (s->ordering == LBLG_ORDER_GIVEN && !perm) return LBLG_ERR_ARG;
   if (s->cost_param < 1 || s->final_seq_node < 1) return LBLG_ERR_ARG;
-  try {
+  return lblg::guarded([&] {
     h->set = *s;
     h->dev.reset();  // a new analysis invalidates the device factor
     h->analyzed = false;
@@ -111,11 +107,7 @@ extern "C" int lblg_analyze(lblg_handle* hh, const lblg_settings* s, const int* 
     h->analyzed = lblg::analyze(A, order.data(), extra, opt, h->sym);
     h->factored = false;
     return h->analyzed ? LBLG_OK : LBLG_ERR_ARG;
-  } catch (const std::invalid_argument&) {
-    return LBLG_ERR_ARG;
-  } catch (const std::bad_alloc&) {
-    return LBLG_ERR_NOMEM;
-  }
+  });
 }
 
 extern "C" int64_t lblg_symbolic_scalar(const lblg_handle* hh, int which) {
@@ -140,7 +132,7 @@ extern "C" int64_t lblg_symbolic_ints(const lblg_handle* hh, int which, int* dst
   if (!h || !h->analyzed) return LBLG_ERR_STATE;
   const lblg::Symbolic& S = h->sym;
   const std::vector<int>* v = nullptr;
-  std::vector<int> tmp;
+  int64_t count = -1;  // entries to copy (-1: all)
   switch (which) {
     case 0: v = &S.perm; break;
     case 1: v = &S.iperm; break;
@@ -149,15 +141,16 @@ extern "C" int64_t lblg_symbolic_ints(const lblg_handle* hh, int which, int* dst
     case 4: v = &S.super; break;
     case 5: v = &S.col2sup; break;
     case 6: v = &S.sparent; break;
-    case 7: tmp.assign(S.s.begin(), S.s.begin() + S.pi[S.nsuper]); v = &tmp; break;
+    case 7: v = &S.s; count = S.pi[S.nsuper]; break;
     case 8: v = &S.lbc.level_ptr; break;
     case 9: v = &S.lbc.par_ptr; break;
-    case 10: tmp.assign(S.lbc.par_set.begin(), S.lbc.par_set.begin() + S.lbc.par_ptr.back()); v = &tmp; break;
+    case 10: v = &S.lbc.par_set; count = S.lbc.par_ptr.back(); break;
     case 11: v = &S.extra_cols; break;
     default: return LBLG_ERR_ARG;
   }
-  if (dst) std::memcpy(dst, v->data(), v->size() * sizeof(int));
-  return (int64_t)v->size();
+  if (count < 0) count = (int64_t)v->size();
+  if (dst) std::memcpy(dst, v->data(), (size_t)count * sizeof(int));
+  return count;
 }
 
 extern "C" int64_t lblg_symbolic_longs(const lblg_handle* hh, int which, int64_t* dst) {

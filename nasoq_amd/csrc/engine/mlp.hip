@@ -18,6 +18,7 @@
 #include <string>
 #include <vector>
 
+#include "capi_guard.hpp"
 #include "engine/device_util.hpp"
 #include "lblg.h"
 
@@ -358,31 +359,13 @@ struct Mlp {
 
 }  // namespace lblg
 
+using lblg::guarded;
 using lblg::Mlp;
-
-namespace lblg {
-void set_last_error(const char* what);  // capi_numeric.cpp (lblg_last_error)
-}
-
-namespace {
-template <typename F>
-int mlp_guard(F f) {
-  try {
-    return f();
-  } catch (const std::bad_alloc&) {
-    lblg::set_last_error("mlp: allocation failed");
-    return LBLG_ERR_NOMEM;
-  } catch (const std::exception& e) {
-    lblg::set_last_error(e.what());
-    return LBLG_ERR_DEVICE;
-  }
-}
-}  // namespace
 
 extern "C" int lblg_mlp_create(lblg_mlp** out, int in, int h1, int h2, int nout, uint64_t seed, int max_batch) {
   if (!out || in < 1 || h1 < 1 || h2 < 1 || nout < 1 || max_batch < 1) return LBLG_ERR_ARG;
   *out = nullptr;
-  return mlp_guard([&] {
+  return guarded([&] {
     Mlp* m = new Mlp;
     try {
       m->in = in;
@@ -456,7 +439,7 @@ extern "C" int lblg_mlp_get_params(lblg_mlp* mm, float* p) {
 extern "C" int lblg_mlp_set_params(lblg_mlp* mm, const float* p) {
   Mlp* m = reinterpret_cast<Mlp*>(mm);
   if (!m || !p) return LBLG_ERR_ARG;
-  return mlp_guard([&] {
+  return guarded([&] {
     if (hipMemcpy(m->P, p, sizeof(float) * m->np, hipMemcpyHostToDevice) != hipSuccess)
       throw std::runtime_error("upload");
     lblg::k_to_bf16<<<lblg::ew_grid(m->np), 256, 0, m->st>>>(m->P, m->Pb, m->np);
@@ -471,7 +454,7 @@ extern "C" int lblg_mlp_set_params(lblg_mlp* mm, const float* p) {
 extern "C" int lblg_mlp_gradients(lblg_mlp* mm, const float* X, const float* Y, int batch, float* grad, float* loss) {
   Mlp* m = reinterpret_cast<Mlp*>(mm);
   if (!m || !X || !Y || !grad || batch < 1 || batch > m->bmax) return LBLG_ERR_ARG;
-  return mlp_guard([&] {
+  return guarded([&] {
     MLP_HIP(hipMemcpyAsync(m->X, X, sizeof(float) * batch * m->in, hipMemcpyHostToDevice, m->st));
     MLP_HIP(hipMemcpyAsync(m->Y, Y, sizeof(float) * batch * m->out, hipMemcpyHostToDevice, m->st));
     m->forward(batch);
@@ -489,7 +472,7 @@ extern "C" int lblg_mlp_train(lblg_mlp* mm, const float* X, const float* Y, int 
                               float lr, uint64_t seed, float* last_loss) {
   Mlp* m = reinterpret_cast<Mlp*>(mm);
   if (!m || !X || !Y || nsamples < 1 || batch < 1 || batch > m->bmax || epochs < 0) return LBLG_ERR_ARG;
-  return mlp_guard([&] {
+  return guarded([&] {
     std::vector<int> order(nsamples);
     for (int i = 0; i < nsamples; ++i) order[i] = i;
     std::mt19937_64 rng(seed);
@@ -524,7 +507,7 @@ extern "C" int lblg_mlp_train(lblg_mlp* mm, const float* X, const float* Y, int 
 extern "C" int lblg_mlp_predict(lblg_mlp* mm, const float* X, int nsamples, float* P) {
   Mlp* m = reinterpret_cast<Mlp*>(mm);
   if (!m || !X || !P || nsamples < 1) return LBLG_ERR_ARG;
-  return mlp_guard([&] {
+  return guarded([&] {
     for (int s0 = 0; s0 < nsamples; s0 += m->bmax) {
       const int B = std::min(m->bmax, nsamples - s0);
       MLP_HIP(hipMemcpyAsync(m->X, X + (size_t)s0 * m->in, sizeof(float) * B * m->in, hipMemcpyHostToDevice, m->st));
@@ -539,7 +522,7 @@ extern "C" int lblg_mlp_predict(lblg_mlp* mm, const float* X, int nsamples, floa
 
 extern "C" int lblg_selftest_mfma_bf16(const float* A, const float* B, float* C) {
   if (!A || !B || !C) return LBLG_ERR_ARG;
-  return mlp_guard([&] {
+  return guarded([&] {
     float* d = nullptr;  // A, B, C: 256 floats each
     MLP_HIP(hipMalloc(&d, 3 * 256 * sizeof(float)));
     struct Free {

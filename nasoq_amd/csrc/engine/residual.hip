@@ -14,9 +14,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
-#include <new>
 #include <stdexcept>
 
+#include "capi_guard.hpp"
 #include "engine/device.hpp"
 #include "engine/device_util.hpp"
 #include "engine/handle.hpp"
@@ -25,7 +25,6 @@
 
 namespace lblg {
 
-void set_last_error(const char* what);  // capi_numeric.cpp
 
 constexpr int RES_BLOCKS = 1024;                      // workgroups of the partial-sum launch, at most
 constexpr int RES_PART = RES_BLOCKS * 3 * MAX_RHS;    // partial sums: [block][|r|, |x|, |b|][column]
@@ -132,22 +131,6 @@ static double* owned_alloc(DeviceFactor& D, int64_t count) {
   return static_cast<double*>(p);
 }
 
-template <typename F>
-static int guard(F f) {
-  try {
-    return f();
-  } catch (const std::bad_alloc&) {
-    set_last_error("allocation failed");
-    return LBLG_ERR_NOMEM;
-  } catch (const std::invalid_argument& e) {
-    set_last_error(e.what());
-    return LBLG_ERR_ARG;
-  } catch (const std::exception& e) {
-    set_last_error(e.what());
-    return LBLG_ERR_DEVICE;
-  }
-}
-
 }  // namespace lblg
 
 using lblg::DeviceFactor;
@@ -158,7 +141,7 @@ extern "C" int lblg_backward_error_device(lblg_handle* hh, int nrhs, const doubl
   Handle* h = reinterpret_cast<Handle*>(hh);
   const int rc = lblg::residual_args(h, nrhs, dB, ldb, dX, ldx, d_err);
   if (rc != LBLG_OK) return rc;
-  return lblg::guard([&] {
+  return lblg::guarded([&] {
     DeviceFactor& D = *h->dev;
     if (!D.res_part) D.res_part = lblg::owned_alloc(D, lblg::RES_PART);
     lblg::launch_residual(D, nrhs, dB, ldb, dX, ldx, D.res_part, nullptr, d_err, D.stream);
@@ -171,7 +154,7 @@ extern "C" int lblg_residual_norms(lblg_handle* hh, int nrhs, const double* B, i
   Handle* h = reinterpret_cast<Handle*>(hh);
   const int rc = lblg::residual_args(h, nrhs, B, ldb, X, ldx, norms);
   if (rc != LBLG_OK) return rc;
-  return lblg::guard([&] {
+  return lblg::guarded([&] {
     DeviceFactor& D = *h->dev;
     const int n = h->n;
     hipStream_t st = D.stream;
@@ -246,7 +229,7 @@ extern "C" int lblg_backward_error_device_noalloc(lblg_handle* hh, int nrhs, con
   }
   const int rc = lblg::residual_args(h, nrhs, dB, ldb, dX, ldx, d_err);
   if (rc != LBLG_OK) return rc;
-  return lblg::guard([&] {
+  return lblg::guarded([&] {
     DeviceFactor& D = *h->dev;
     int dev = -1;
     if (hipStreamGetDevice(D.stream, &dev) != hipSuccess) throw std::runtime_error("no-alloc residual: stream device");

@@ -76,3 +76,17 @@ def test_tuning_knobs_on_the_host():
     with _pt.raises(RuntimeError):
         s.set_tuning(group_w=8)
     s.close()
+
+
+def test_exceptions_end_at_the_c_abi(tmp_path):
+    # every host entry point under a failing allocation and under exceptions
+    # of other types: a status, no abort, and the handle works afterwards
+    import pytest as _pt
+    exe = str(tmp_path / "alloc_failures")
+    libdir = os.path.dirname(_lib.LIB_PATH)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "include"),
+                    os.path.join(ROOT, "tests", "cpp", "alloc_failures.cpp"), "-o", exe, "-L", libdir, "-llblg",
+                    "-Wl,-rpath," + libdir, "-Wl,-rpath,/opt/rocm/lib", "-Wl,-rpath-link,/opt/rocm/lib"], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    last = out.stdout.splitlines()[-1:] + [l for l in out.stdout.splitlines() if l.startswith("FAIL")][:5]
+    assert out.returncode == 0, (out.returncode, last, out.stderr[-300:])
