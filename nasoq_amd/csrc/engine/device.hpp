@@ -218,6 +218,7 @@ struct DeviceFactor {
   };
   GraphCache gfactor, gsolve, gcycle;
   bool graphs = true;       // LBLG_GRAPH=0 turns capture off
+  bool panel_lds = true;         // one-workgroup panels of diagonal blocks that fit: staged in LDS
   bool schur_direct = true;      // 128-tile Schur updates with operands loaded lane by lane (no LDS)
   bool trailing_direct = true;   // the same for the wide panels' trailing updates
   bool strip64 = true;           // the wide panels' strip pre-updates in 64 x 64 tiles

@@ -708,6 +708,7 @@ static void setup(Handle& h) {
     D.ss_max_nnz = h.tune.small_nnz;
     D.graphs = env_int("LBLG_GRAPH", 1) != 0;
     D.schur_direct = env_int("LBLG_SCHUR_DIRECT", 1) != 0;
+    D.panel_lds = env_int("LBLG_PANEL_LDS", 1) != 0;
     D.path_refactor = env_int("LBLG_PATH_REFACTOR", 1) != 0;
     D.trailing_direct = env_int("LBLG_TRAILING_DIRECT", 1) != 0;
     D.strip64 = env_int("LBLG_STRIP_TILE64", 1) != 0;
@@ -837,7 +838,7 @@ static void factor_level(Handle& h, FactorLevel& F, const LevelLists& L, const S
     const int wmax = L.medium_wmax;
     for (int lo = 0;;) {
       const int left = wmax - lo;
-      const int one = one_panel_nb<T>(left), nb = one ? one : PANEL_NB;
+      const int one = D.panel_lds ? one_panel_nb<T>(left) : 0, nb = one ? one : PANEL_NB;
       timed(D, "bk_panel", [&] {
         if (one)
           launch_bk_one(L.medium, L.nmedium, left, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart,

@@ -2,11 +2,14 @@
 oracle, at the edges of their tiles: widths around the panel, sub-block and
 workgroup sizes, with rows below the diagonal block, every step a 1x1 pivot
 in place or one column whose zero diagonal forces a pivot search there."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from nasoq_amd import lbl
 from nasoq_amd import problems as P
+from nasoq_amd._lib import check
 
 from test_gpu_lbl import check_factor
 
@@ -53,6 +56,28 @@ def test_panel_widths(oracle, w, group_w, monkeypatch):
         x = s.solve_only(B[:, 0])
         assert oracle.backward_error(n, Ap, Ai, Ax, x, B[:, 0]) <= 1e-12
         s.close()
+
+
+@pytest.mark.parametrize("w", [65, 97, 321])
+def test_panels_in_memory(oracle, w, monkeypatch):
+    # LBLG_PANEL_LDS=0: panels of 31 to 32 columns in memory, more launches
+    # than the 64-column panels in LDS take
+    monkeypatch.setenv("LBLG_GROUP_W", "4096")
+    launches = {}
+    for lds in (1, 0):
+        monkeypatch.setenv("LBLG_PANEL_LDS", str(lds))
+        for zero_at in ((), (0,), (17, w - 1)):
+            s, n, Ap, Ai, Ax, B = run(oracle, w, 37, zero_at)
+            check_factor(oracle, s, n, Ap, Ai, Ax, 0.0)
+            x = s.solve_only(B[:, 0])
+            assert oracle.backward_error(n, Ap, Ai, Ax, x, B[:, 0]) <= 1e-12
+            check(s.lib.lblg_set_kernel_timing(s.h, 1), "timing")
+            s.refactor_resident()
+            ms, count = ctypes.c_double(), ctypes.c_int64()
+            check(s.lib.lblg_kernel_time(s.h, b"bk_panel", ctypes.byref(ms), ctypes.byref(count)), "kernel time")
+            launches[lds] = count.value
+            s.close()
+    assert launches[0] > launches[1] > 0, launches
 
 
 @pytest.mark.parametrize("group_w", [64, 4096])
