@@ -236,7 +236,9 @@ __global__ __launch_bounds__(NT) void k_bk_wide(WideSn sn, PanelList pl, int G, 
     Wp = Wbase + sn.woff;
   }
   const T* Pp = Wp + (int64_t)w * wcols;  // this panel's columns with the block's earlier panels applied
-  T* scr = Wp + (int64_t)w * wcols + (ONE ? 0 : (int64_t)r * nb);
+  // scratch of the interchanges; one workgroup: in W's place, whose columns
+  // are written after them (at most min(nb, w) moved indices squared)
+  T* scr = ONE ? Wp : Wp + (int64_t)w * wcols + (int64_t)r * nb;
   const int k0 = kpos[s];
   if (k0 >= w) return;
   // sub > 0: this panel continues the block of panels that started at K0.
@@ -1029,7 +1031,7 @@ __global__ __launch_bounds__(NT) void k_bk_wide(WideSn sn, PanelList pl, int G, 
         const int m = idx / nMa, q = idx % nMa;
         if (m >= q) sym(Ml[m], Ml[q]) = scr[idx];
       }
-      __syncthreads();  // the panel's original columns are read: L may go over them
+      __syncthreads();  // the panel's original columns and the scratch are read: L and W may go over them
     }
   } else {
     T* S1 = scr;                                  // [nMa][nt]

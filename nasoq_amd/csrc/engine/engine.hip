@@ -404,7 +404,7 @@ static void setup(Handle& h) {
         if (w <= group_w) {
           F.medium.push_back(s);
           D.s_kind[s] = 1;
-          wsum += (int64_t)w * ONE_WCOLS + ONE_WCOLS * ONE_WCOLS + 16;
+          wsum += (int64_t)w * ONE_WCOLS;
         } else {
           // cooperative panel over G workgroups, <= WIDE_ROWS far rows each
           // (the diagonal block below the panel and the off-diagonal rows);

@@ -81,7 +81,7 @@ void launch_bk_wide(const WideSn& sn, int G, int nt, int nb, int sub, int wcols,
 // One-workgroup panels of the listed supernodes, all with at most `rows`
 // diagonal-block rows left: one_panel_nb<T>(rows) columns each (0: too many
 // rows; those take launch_bk_panel).
-constexpr int ONE_WCOLS = 64;  // columns of their W workspace
+constexpr int ONE_WCOLS = 64;  // columns of their workspace (W; the memory form: W, t0, t1)
 template <typename T>
 int one_panel_nb(int rows);
 template <typename T>
