@@ -539,8 +539,8 @@ static void setup(Handle& h) {
   D.woff = dupload(D, woff);
   D.kpos = dalloc<int>(D, ns);
   D.kstart = dalloc<int>(D, ns);
-  D.sync = dalloc<int>(D, std::max<int64_t>(ns, 2));
-  launch_fill_int(D.sync, (int)std::max<int64_t>(ns, 2), 0, D.stream);  // the wide panel's two counters start at 0
+  D.sync = dalloc<int>(D, 2);
+  launch_fill_int(D.sync, 2, 0, D.stream);  // the wide panel's two counters start at 0
   D.wide_par = 0;
   D.ll = reinterpret_cast<uint64_t*>(dalloc<double>(D, LL_WORDS));
   launch_fill(reinterpret_cast<double*>(D.ll), LL_WORDS, 0.0, D.stream);
@@ -844,8 +844,8 @@ static void factor_level(Handle& h, FactorLevel& F, const LevelLists& L, const S
           launch_bk_one(L.medium, L.nmedium, left, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart,
                         D.status, st);
         else
-          launch_bk_panel(L.medium, L.nmedium, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart, D.sync,
-                          D.status, st);
+          launch_bk_panel(L.medium, L.nmedium, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart, D.status,
+                          st);
       });
       if (left <= nb) break;
       lo += nb - 1;

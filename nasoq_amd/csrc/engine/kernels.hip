@@ -376,36 +376,28 @@ void launch_bk_small(const int* list, int count, int wmax, const SnArgs& a, T* v
 // (k_trailing).  Interchanges are applied to all earlier columns of L and to
 // the columns of the rows below the diagonal block (the column permutation
 // of LAPACKE_dlapmt at parallel_blocked_ldlt_02.cpp:164-165), so no separate
-// permutation pass is needed.  G workgroups cooperate on one supernode.
+// permutation pass is needed.  One workgroup per supernode, the panel in
+// memory: for diagonal blocks with more rows left than the LDS form holds
+// (bk_wide.hip, ONE).
 //
 // Per-supernode workspace at W + woff[s]:  Wp (w x NB, ld w) | t0 (w) | t1 (w)
-//                                         | part (2 G doubles) | parti (2 G ints)
-//
-// This form, with the panel in memory, takes the diagonal blocks with more
-// rows left than a one-workgroup panel's LDS holds (bk_wide.hip, ONE).
 // --------------------------------------------------------------------------
 constexpr int PANEL_UF = 8;  // left-looking terms whose loads are issued together
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const int* super,
-                                                  const int64_t* pi, const int64_t* px, T* valL,
-                                                  T* dval, int* perm_piv, T* Wbase,
-                                                  const int64_t* woff, int* kpos, int* kstart,
-                                                  int* sync, int n, int* status) {
+__global__ __launch_bounds__(256) void k_bk_panel(const int* list, const int* super, const int64_t* pi,
+                                                  const int64_t* px, T* valL, T* dval, int* perm_piv, T* Wbase,
+                                                  const int64_t* woff, int* kpos, int* kstart, int n,
+                                                  int* status) {
   __shared__ double sv[8];
   __shared__ int si[8];
-  const int sidx = blockIdx.x / G, g = blockIdx.x % G;
-  const int s = list[sidx];
+  const int s = list[blockIdx.x], t = threadIdx.x;
   const int c0 = super[s], w = super[s + 1] - c0;
   const int64_t r = pi[s + 1] - pi[s];
   T* A = valL + px[s];
   T* Wp = Wbase + woff[s];
-  T* part = Wp + (int64_t)w * PANEL_NB + 2 * (int64_t)w;  // column maxima (exact in T: magnitudes of T values)
-  int* parti = reinterpret_cast<int*>(part + 2 * G);
-  int* ctr = sync + sidx;
-  const int gt = g * 256 + threadIdx.x, GT = G * 256;
   const int k0 = kpos[s];
-  if (k0 >= w) return;  // whole group returns together (k0 is uniform)
+  if (k0 >= w) return;  // uniform
   const bool last = (w - k0) <= PANEL_NB;
   T* t0 = Wp + (int64_t)w * PANEL_NB;  // indexed by row i >= k0
   T* t1 = Wp + (int64_t)w * PANEL_NB + w;
@@ -427,13 +419,12 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
     for (; j < k; ++j) v -= A[(int64_t)j * r + i] * Wp[(int64_t)(j - k0) * w + q];
     return v;
   };
-  int epoch = 0;
   int k = k0;
   while (k < w && (last || k - k0 < PANEL_NB - 1)) {
-    // ---- phase A: updated column k for own rows, local argmax
+    // ---- phase A: updated column k, its largest candidate
     double bv = -1.0;
     int bi = 0x7fffffff;
-    for (int i = k + gt; i < w; i += GT) {
+    for (int i = k + t; i < w; i += 256) {
       const T v = left_update(AA(i, k), i, k, k);
       t0[i] = v;
       if (i > k) {
@@ -442,20 +433,9 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
         better(bv, bi, av, i);
       }
     }
-    block_argmax(bv, bi, sv, si);
-    if (G > 1 && threadIdx.x == 0) {
-      part[g] = (T)bv;
-      parti[g] = bi;
-    }
-    group_barrier(ctr, G, epoch, status);
-    double colmax = -1.0;
-    int imax = 0x7fffffff;
-    if (G > 1) {
-      for (int q = 0; q < G; ++q) better(colmax, imax, part[q], parti[q]);
-    } else {  // the block maximum in T, as the cross-group exchange stores it
-      colmax = (double)(T)bv;
-      imax = bi;
-    }
+    block_argmax(bv, bi, sv, si);  // ends with a barrier
+    double colmax = bv;  // a magnitude of a T value: exact in T
+    int imax = bi;
     if (k == w - 1 || colmax < 0) {
       colmax = 0.0;
       imax = k;
@@ -470,7 +450,7 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
       // ---- phase B: updated column imax, row maximum
       double rv = -1.0;
       int ri = 0x7fffffff;
-      for (int i = k + gt; i < w; i += GT) {
+      for (int i = k + t; i < w; i += 256) {
         const T v = left_update((i < imax) ? AA(imax, i) : AA(i, imax), i, imax, k);
         t1[i] = v;
         if (i != imax) {
@@ -480,20 +460,7 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
         }
       }
       block_argmax(rv, ri, sv, si);
-      if (G > 1 && threadIdx.x == 0) {
-        part[G + g] = (T)rv;
-        parti[G + g] = ri;
-      }
-      group_barrier(ctr, G, epoch, status);
-      double rowmax = -1.0;
-      int rj = 0x7fffffff;
-      if (G > 1) {
-        for (int q = 0; q < G; ++q) better(rowmax, rj, part[G + q], parti[G + q]);
-      } else {
-        rowmax = (double)(T)rv;
-        rj = ri;
-      }
-      if (rowmax < 0) rowmax = 0.0;
+      const double rowmax = fmax(rv, 0.0);
       if (absakk >= BK_ALPHA * colmax * (colmax / rowmax)) {
         kp = k;
       } else if (fabs(t1[imax]) >= BK_ALPHA * rowmax) {
@@ -507,26 +474,26 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
     const int kk = k + kstep - 1;
     const bool swap = kp != kk;
     // ---- phase C: interchange, W and L columns
-    if (zero && gt == 0) atomicOr(status, 1);
+    if (zero && t == 0) atomicOr(status, 1);
     if (swap) {
       // rows kk/kp of the earlier L columns and of the panel's W columns
-      for (int j = gt; j < k; j += GT) {
+      for (int j = t; j < k; j += 256) {
         const T x = AA(kk, j);
         AA(kk, j) = AA(kp, j);
         AA(kp, j) = x;
       }
-      for (int j = k0 + gt; j < k; j += GT) {
+      for (int j = k0 + t; j < k; j += 256) {
         const T x = WW(kk, j);
         WW(kk, j) = WW(kp, j);
         WW(kp, j) = x;
       }
       // columns kk/kp of the rows below the diagonal block
-      for (int64_t q = w + gt; q < r; q += GT) {
+      for (int64_t q = w + t; q < r; q += 256) {
         const T x = AA(q, kk);
         AA(q, kk) = AA(q, kp);
         AA(q, kp) = x;
       }
-      if (gt == 0) {
+      if (t == 0) {
         const int tp = perm_piv[c0 + kk];
         perm_piv[c0 + kk] = perm_piv[c0 + kp];
         perm_piv[c0 + kp] = tp;
@@ -550,7 +517,7 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
       const T tt = (T)1 / (d11 * d22 - (T)1);
       d21 = tt / d21;
     }
-    for (int i = k + gt; i < w; i += GT) {
+    for (int i = k + t; i < w; i += 256) {
       const int si2 = !swap ? i : (i == kk ? kp : (i == kp ? kk : i));
       if (swap) {
         if (i == kk) AA(kp, kp) = AA(kk, kk);
@@ -586,10 +553,10 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
         }
       }
     }
-    group_barrier(ctr, G, epoch, status);
+    __syncthreads();
     k += kstep;
   }
-  if (gt == 0) {
+  if (t == 0) {
     kstart[s] = k0;
     kpos[s] = k;
   }
@@ -597,10 +564,10 @@ __global__ __launch_bounds__(256) void k_bk_panel(const int* list, int G, const 
 
 template <typename T>
 void launch_bk_panel(const int* list, int count, const SnArgs& a, T* valL, T* dval, int* perm_piv, T* W,
-                     const int64_t* woff, int* kpos, int* kstart, int* sync, int* status, hipStream_t st) {
+                     const int64_t* woff, int* kpos, int* kstart, int* status, hipStream_t st) {
   if (count <= 0) return;
-  k_bk_panel<T><<<count, 256, 0, st>>>(list, 1, a.super, a.pi, a.px, valL, dval, perm_piv, W, woff, kpos, kstart,
-                                       sync, a.n, status);
+  k_bk_panel<T><<<count, 256, 0, st>>>(list, a.super, a.pi, a.px, valL, dval, perm_piv, W, woff, kpos, kstart, a.n,
+                                       status);
   HIP_LAUNCH_CHECK("bk_panel");
 }
 
@@ -2343,7 +2310,7 @@ void launch_k0(int n, int64_t nnzf, const int* rp, const int64_t* src, const dou
   template void launch_reset_supernodes<T>(const int*, int, const SnArgs&, T*, T*, int*, hipStream_t);          \
   template void launch_bk_small<T>(const int*, int, int, const SnArgs&, T*, T*, int*, int*, hipStream_t);      \
   template void launch_bk_panel<T>(const int*, int, const SnArgs&, T*, T*, int*, T*, const int64_t*, int*, int*,  \
-                                   int*, int*, hipStream_t);                                       \
+                                   int*, hipStream_t);                                             \
   template void launch_trailing<T>(const int*, int, int, int, const SnArgs&, T*, const T*, const int64_t*,      \
                                    const int*, const int*, hipStream_t);                                       \
   template void launch_offdiag<T>(const int*, int, int, const int*, const int*, int, const SnArgs&, T*,      \

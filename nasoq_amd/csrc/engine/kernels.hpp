@@ -54,7 +54,7 @@ void launch_bk_small(const int* list, int count, int wmax, const SnArgs& a, T* v
 // one workgroup per listed supernode, panels of PANEL_NB columns in memory
 template <typename T>
 void launch_bk_panel(const int* list, int count, const SnArgs& a, T* valL, T* dval, int* perm_piv, T* W,
-                     const int64_t* woff, int* kpos, int* kstart, int* sync, int* status, hipStream_t st);
+                     const int64_t* woff, int* kpos, int* kstart, int* status, hipStream_t st);
 // wide panels with flag-in-word exchange (bk_wide.hip)
 constexpr int WIDE_NB = 64;         // panel width
 constexpr int WIDE_ROWS = 192;      // far rows per workgroup (256-thread workgroups)
