@@ -94,3 +94,77 @@ def test_panel_float(oracle, group_w, monkeypatch):
         x = s.solve_only(B[:, 0])
         assert oracle.backward_error(n, Ap, Ai, Ax, x, B[:, 0]) <= 1e-12
         s.close()
+
+
+def mixed_blocks(widths, m2, kind, seed):
+    """Dense diagonal blocks of the given widths and one 70 wide, with m2 dense
+    common rows below: a supernode per block, all in one level, and one of
+    70 + m2 columns.  kind: the columns whose diagonal is 0 ("none", "first",
+    "middle", "last"), "some" every 23rd, or "random" for N(0, 1) blocks."""
+    rng = np.random.default_rng(seed)
+    widths = list(widths) + [70]
+    n1 = sum(widths)
+    n = n1 + m2
+    K = np.zeros((n, n))
+    c0 = 0
+    for w in widths:
+        b = rng.standard_normal((w, w)) * (1.0 if kind == "random" else 0.3)
+        b = np.tril(b) + np.tril(b, -1).T
+        if kind != "random":
+            d = np.full(w, float(w))
+            d[{"none": [], "first": [0], "middle": [w // 2], "last": [w - 1], "some": np.arange(7, w, 23)}[kind]] = 0.0
+            np.fill_diagonal(b, d)
+        K[c0:c0 + w, c0:c0 + w] = b
+        c0 += w
+    K[n1:, :n1] = rng.standard_normal((m2, n1))
+    K[n1:, n1:] = -np.diag(rng.uniform(1.0, 2.0, m2))
+    low = np.tril(np.ones((n, n), bool))
+    low[n1:, n1:] = np.eye(m2, dtype=bool)
+    c0 = 0
+    for w in widths:
+        low[c0 + w:n1, c0:c0 + w] = False
+        c0 += w
+    cols, rows = np.nonzero(low.T)
+    Ap = np.r_[0, np.cumsum(np.bincount(cols, minlength=n))].astype(np.int32)
+    return n, Ap, rows.astype(np.int32), K[rows, cols], rng.uniform(-1.0, 1.0, n)
+
+
+def analyzed(n, Ap, Ai, Ax, precision, wmax):
+    s = lbl.SolverSettings(n, Ap, Ai, Ax)
+    s.reg_diag, s.regularization, s.precision = 1e-9, 0, precision
+    s.n_relax, s.z_relax = [0, 0, 0], [0.0, 0.0, 0.0]
+    assert s.symbolic_analysis(perm=np.arange(n, dtype=np.int32)) == 1
+    assert s.sym_scalar("max_sup_wid") == wmax
+    return s
+
+
+# one-workgroup panels: 64 columns up to 256 rows left, then 32 up to 480 (FP64)
+# / 64 up to 512 (FP32), 16 up to 976 / 32 up to 992, beyond that in memory
+@pytest.mark.parametrize("kind", ["none", "first", "middle", "last", "some", "random"])
+@pytest.mark.parametrize("widths", [(256, 65, 257), (480, 130, 481), (976, 200), (977, 65, 300), (1010, 513),
+                                    (95, 97, 112)])
+def test_panel_shapes_mixed(oracle, widths, kind, monkeypatch):
+    monkeypatch.setenv("LBLG_GROUP_W", "4096")
+    n, Ap, Ai, Ax, b = mixed_blocks(widths, 7, kind, seed=max(widths))
+    print(f"case panel shapes widths={widths} kind={kind}", flush=True)
+    s = analyzed(n, Ap, Ai, Ax, lbl.F64, max(widths))
+    assert s.numerical_factorization() == 1
+    check_factor(oracle, s, n, Ap, Ai, Ax, 0.0)
+    x = s.solve_only(b)
+    assert oracle.backward_error(n, Ap, Ai, Ax, x, b) <= 1e-12
+    s.close()
+
+
+@pytest.mark.parametrize("kind", ["some", "random"])
+@pytest.mark.parametrize("widths", [(512, 65, 513), (992, 300, 993), (1010, 97)])
+def test_panel_shapes_float(oracle, widths, kind, monkeypatch):
+    # the FP32 factor on the same shapes, refined to an FP64 backward error
+    monkeypatch.setenv("LBLG_GROUP_W", "4096")
+    n, Ap, Ai, Ax, b = mixed_blocks(widths, 7, kind, seed=max(widths))
+    print(f"case float panel shapes widths={widths} kind={kind}", flush=True)
+    s = analyzed(n, Ap, Ai, Ax, lbl.F32, max(widths))
+    s.target_bwd_err = 1e-12
+    assert s.numerical_factorization() == 1
+    x = s.solve_only(b)
+    assert oracle.backward_error(n, Ap, Ai, Ax, x, b) <= 1e-12
+    s.close()
