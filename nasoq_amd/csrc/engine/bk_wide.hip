@@ -172,6 +172,13 @@ __device__ inline int far_phys(int a, int fstart, const unsigned* mbits, const i
   return a;
 }
 
+// Waves per SIMD to compile for: the FP32 panels of many supernodes share a
+// CU, four workgroups with 128 registers (two spilled) instead of three.
+template <typename T, int NT, int NBM, bool ONE>
+constexpr int panel_waves() {
+  return ONE && NT == 256 && NBM == 32 && sizeof(T) == 4 ? 4 : 1;
+}
+
 // NT threads per workgroup: waves 0 .. NT/64 - 2 own one far row per
 // thread (WCH = NT - 64 rows per workgroup), the last wave computes the
 // diagonal rows; NBM is the widest panel the launch takes.
@@ -185,17 +192,16 @@ __device__ inline int far_phys(int a, int fstart, const unsigned* mbits, const i
 // the diagonal block (at most WCH), the rows below it are left to
 // k_offdiag, and every exchange stays inside the workgroup.
 template <typename T, int NT, int NBM, bool ONE>
-__global__ __launch_bounds__(NT) void k_bk_wide(WideSn sn, PanelList pl, int G, int nb, int sub, int wcols, T* valL,
-                                                 T* dval, int* perm_piv, T* Wbase, int* kpos, int* kstart, int* sync,
-                                                 int* sync_next, uint64_t* ll, uint32_t ebase, int n,
-                                                 int* status) {
+__global__ __launch_bounds__(NT, (panel_waves<T, NT, NBM, ONE>())) void k_bk_wide(
+    WideSn sn, PanelList pl, int G, int nb, int sub, int wcols, T* valL, T* dval, int* perm_piv, T* Wbase, int* kpos,
+    int* kstart, int* sync, int* sync_next, uint64_t* ll, uint32_t ebase, int n, int* status) {
   constexpr int NW = NT / 64;                   // waves; wave NW - 1 holds the diagonal rows
   constexpr int WCH = NT - 64;                  // far rows per workgroup
   constexpr int WLDA = NBM + 1;                 // padded row length of the diagonal rows
   constexpr int WLDC = WCH + 16;                // padded column length of the far rows: the k-groups of an MFMA
                                                 // operand read fall into different banks
   constexpr int MBITS_WORDS = (ONE ? 1 : 256) * WCH / 32;  // moved-far-row bitmap
-  static_assert(NBM <= WNB && NT % 64 == 0 && NT >= 256 && WCH % 32 == 0, "wide panel launch shape");
+  static_assert(NBM <= WNB && NT % 64 == 0 && NT >= (ONE ? 128 : 256) && WCH % 32 == 0, "wide panel launch shape");
   __shared__ T LC[NBM * WLDC];      // own far rows, column-major [column][row]
   __shared__ T Ad[NBM * WLDA];      // diagonal rows: L below the diagonal and W(j, c) at (c, j) above it
                                     // (eliminated columns c) | symmetric A (pending)
@@ -1147,36 +1153,64 @@ template void launch_bk_wide<float>(const WideSn&, int, int, int, int, int, int,
 // remaining rows: 256 threads and 64 columns up to 256 rows, 512 threads up
 // to 448 far rows (32 FP64 or 64 FP32 columns), 1024 threads up to 960 far
 // rows (16 or 32 columns): the same LDS (far rows x columns) in all three.
+//
+// A 64-column FP64 panel takes 146 KB of LDS, so a CU runs one (FP32: two).
+// Launches of more panels than that take 32 columns, where 33 KB (128
+// threads, up to 96 rows) or 66 KB (up to 224 rows) let a CU run four or two
+// side by side.  All panels of one factorization, us, 64 columns / 32 columns
+// (and 31-column panels with up to four workgroups a CU before): 512 blocks
+// 65 wide, accepted in place 149 / 101 (274), searched at every column
+// 440 / 265 (324); 1024: 278 / 117 (331), 852 / 290 (392); 512 blocks 150
+// wide 325 / 252 (705), 1271 / 707 (826); FP32, 1024 blocks 65 wide
+// 177 / 114 (316), 506 / 288 (376).  Up to one panel per CU (FP32: two) the
+// 64-column panels win: 256 blocks 65 wide take 85 us.
+struct OneShape {
+  int nt, nb;  // threads, columns (0: too many rows)
+};
 template <typename T>
-int one_panel_nb(int rows) {
-  constexpr int N0 = 64, N1 = sizeof(T) == 8 ? 32 : 64, N2 = sizeof(T) == 8 ? 16 : 32;
-  if (rows <= N0 + 192) return N0;
-  if (rows <= N1 + 448) return N1;
-  if (rows <= N2 + 960) return N2;
-  return 0;
+static OneShape one_shape(int rows, int count) {
+  constexpr int CUS = 256, N1 = sizeof(T) == 8 ? 32 : 64, N2 = sizeof(T) == 8 ? 16 : 32;
+  if (count > CUS * (sizeof(T) == 8 ? 1 : 2)) {
+    if (rows <= 32 + 64) return {128, 32};
+    if (rows <= 32 + 192) return {256, 32};
+  }
+  if (rows <= 64 + 192) return {256, 64};
+  if (rows <= N1 + 448) return {512, N1};
+  if (rows <= N2 + 960) return {1024, N2};
+  return {0, 0};
 }
-template int one_panel_nb<double>(int);
-template int one_panel_nb<float>(int);
+template <typename T>
+int one_panel_nb(int rows, int count) {
+  return one_shape<T>(rows, count).nb;
+}
+template int one_panel_nb<double>(int, int);
+template int one_panel_nb<float>(int, int);
 
+template <typename T, int NT, int NBM>
+static void launch_one(const PanelList& pl, int count, T* valL, T* dval, int* perm_piv, T* W, int* kpos, int* kstart,
+                       int n, int* status, hipStream_t st) {
+  int* const nosync = nullptr;
+  uint64_t* const noll = nullptr;
+  k_bk_wide<T, NT, NBM, true><<<count, NT, 0, st>>>(WideSn{}, pl, 1, NBM, 0, ONE_WCOLS, valL, dval, perm_piv, W, kpos,
+                                                    kstart, nosync, nosync, noll, 0u, n, status);
+}
 template <typename T>
 void launch_bk_one(const int* list, int count, int rows, const SnArgs& a, T* valL, T* dval, int* perm_piv, T* W,
                    const int64_t* woff, int* kpos, int* kstart, int* status, hipStream_t st) {
   if (count <= 0) return;
   constexpr int N1 = sizeof(T) == 8 ? 32 : 64, N2 = sizeof(T) == 8 ? 16 : 32;
-  const int nb = one_panel_nb<T>(rows);
+  const OneShape sh = one_shape<T>(rows, count);
   const PanelList pl{list, a.super, a.pi, a.px, woff};
-  const WideSn sn{};
-  int* const nosync = nullptr;
-  uint64_t* const noll = nullptr;
-  if (rows <= 64 + 192)
-    k_bk_wide<T, 256, 64, true><<<count, 256, 0, st>>>(sn, pl, 1, nb, 0, ONE_WCOLS, valL, dval, perm_piv, W, kpos,
-                                                      kstart, nosync, nosync, noll, 0u, a.n, status);
-  else if (rows <= N1 + 448)
-    k_bk_wide<T, 512, N1, true><<<count, 512, 0, st>>>(sn, pl, 1, nb, 0, ONE_WCOLS, valL, dval, perm_piv, W, kpos,
-                                                      kstart, nosync, nosync, noll, 0u, a.n, status);
-  else if (rows <= N2 + 960)
-    k_bk_wide<T, 1024, N2, true><<<count, 1024, 0, st>>>(sn, pl, 1, nb, 0, ONE_WCOLS, valL, dval, perm_piv, W, kpos,
-                                                        kstart, nosync, nosync, noll, 0u, a.n, status);
+  if (sh.nt == 128)
+    launch_one<T, 128, 32>(pl, count, valL, dval, perm_piv, W, kpos, kstart, a.n, status, st);
+  else if (sh.nt == 256 && sh.nb == 32)
+    launch_one<T, 256, 32>(pl, count, valL, dval, perm_piv, W, kpos, kstart, a.n, status, st);
+  else if (sh.nt == 256)
+    launch_one<T, 256, 64>(pl, count, valL, dval, perm_piv, W, kpos, kstart, a.n, status, st);
+  else if (sh.nt == 512)
+    launch_one<T, 512, N1>(pl, count, valL, dval, perm_piv, W, kpos, kstart, a.n, status, st);
+  else if (sh.nt == 1024)
+    launch_one<T, 1024, N2>(pl, count, valL, dval, perm_piv, W, kpos, kstart, a.n, status, st);
   else
     throw std::invalid_argument("bk_one: too many rows for a one-workgroup panel");
   HIP_LAUNCH_CHECK("bk_one");

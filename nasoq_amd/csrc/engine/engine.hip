@@ -838,7 +838,7 @@ static void factor_level(Handle& h, FactorLevel& F, const LevelLists& L, const S
     const int wmax = L.medium_wmax;
     for (int lo = 0;;) {
       const int left = wmax - lo;
-      const int one = D.panel_lds ? one_panel_nb<T>(left) : 0, nb = one ? one : PANEL_NB;
+      const int one = D.panel_lds ? one_panel_nb<T>(left, L.nmedium) : 0, nb = one ? one : PANEL_NB;
       timed(D, "bk_panel", [&] {
         if (one)
           launch_bk_one(L.medium, L.nmedium, left, a, valL, dval, D.perm_piv, Wb, D.woff, D.kpos, D.kstart,

@@ -78,12 +78,12 @@ template <typename T>
 void launch_bk_wide(const WideSn& sn, int G, int nt, int nb, int sub, int wcols, int n, T* valL, T* dval,
                     int* perm_piv, T* W, int* kpos, int* kstart, int* sync, int* sync_next, uint64_t* ll,
                     uint32_t ebase, int* status, hipStream_t st);
-// One-workgroup panels of the listed supernodes, all with at most `rows`
-// diagonal-block rows left: one_panel_nb<T>(rows) columns each (0: too many
-// rows; those take launch_bk_panel).
+// One-workgroup panels of `count` listed supernodes, all with at most `rows`
+// diagonal-block rows left: one_panel_nb<T>(rows, count) columns each (0: too
+// many rows; those take launch_bk_panel).
 constexpr int ONE_WCOLS = 64;  // columns of their workspace (W; the memory form: W, t0, t1)
 template <typename T>
-int one_panel_nb(int rows);
+int one_panel_nb(int rows, int count);
 template <typename T>
 void launch_bk_one(const int* list, int count, int rows, const SnArgs& a, T* valL, T* dval, int* perm_piv, T* W,
                    const int64_t* woff, int* kpos, int* kstart, int* status, hipStream_t st);

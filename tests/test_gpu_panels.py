@@ -168,3 +168,42 @@ def test_panel_shapes_float(oracle, widths, kind, monkeypatch):
     x = s.solve_only(b)
     assert oracle.backward_error(n, Ap, Ai, Ax, x, b) <= 1e-12
     s.close()
+
+
+# more panels in a launch than CUs (FP32: twice as many): 32 columns, 128
+# threads up to 96 rows left and 256 threads up to 224
+@pytest.mark.parametrize("precision,count", [(lbl.F64, 257), (lbl.F32, 513)])
+@pytest.mark.parametrize("kind", ["none", "some", "random"])
+@pytest.mark.parametrize("widths", [(65, 96), (97, 79), (224, 127), (225, 65)])
+def test_many_panels(widths, kind, precision, count):
+    print(f"case many panels widths={widths} kind={kind} precision={precision}", flush=True)
+    kinds = []
+    for i, w in enumerate((*widths, 64)):
+        rng = np.random.default_rng(100 * w + i)
+        b = rng.standard_normal((w, w)) * (1.0 if kind == "random" else 0.3)
+        b = np.tril(b) + np.tril(b, -1).T
+        if kind != "random":
+            np.fill_diagonal(b, float(w))
+        if kind == "some":
+            b[np.arange(7, w, 23), np.arange(7, w, 23)] = 0.0
+        iu = np.triu_indices(w)
+        Ap = np.r_[0, np.cumsum(np.arange(w, 0, -1))].astype(np.int32)
+        kinds.append((b, (w, Ap, iu[1].astype(np.int32), np.ascontiguousarray(b[iu]))))
+    pick = [0 if i == count // 2 else 1 for i in range(count)] + [2, 2]
+    s = lbl.BatchSolverSettings([kinds[p][1] for p in pick])
+    s.regularization, s.precision, s.ordering = 0, precision, lbl.ORDER_NATURAL
+    s.req_ref_iter = 0
+    assert s.symbolic_analysis() == 1
+    s.numerical_factorization()
+    x0 = np.random.default_rng(1).uniform(-1.0, 1.0, s.n)
+    rhs = np.concatenate([kinds[p][0] @ x0[o:o + kinds[p][1][0]] for p, o in zip(pick, s.offsets)])
+    x = s.solve_only(rhs)
+    s.close()
+    # one solve without refinement: a backward error of n u times the growth
+    # of the factor's entries, below 100 for these blocks
+    u = 2.0**-53 if precision == lbl.F64 else 2.0**-24
+    for p, o in zip(pick, s.offsets):
+        K, w = kinds[p][0], kinds[p][1][0]
+        r = K @ (x[o:o + w] - x0[o:o + w])
+        bound = 100 * w * u * (np.abs(K).sum(1).max() * np.abs(x[o:o + w]).max() + np.abs(rhs[o:o + w]).max())
+        assert np.abs(r).max() <= bound, (o, w)
