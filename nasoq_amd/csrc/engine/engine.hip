@@ -1389,7 +1389,7 @@ static void apply_solve_t(DeviceFactor& D, const double* in, double* out, int nr
     const int fit_cols = it == D.ssb_cols.begin() ? 0 : *(it - 1);
     timed(D, "solve_batch", [&] {
       launch_solve_batch<T>(D.ssb_sysd, D.ssb_nsys, D.ssb_info, D.ssb_ipx, D.ssb_levptr, D.ssb_mode, fit_cols,
-                            D.ssb_maxlev, a, valL, dval, sin, out, nrhs, active, astride, Z, st);
+                            D.ssb_cols.back(), D.ssb_maxlev, a, valL, dval, sin, out, nrhs, active, astride, Z, st);
     });
     if (scaled) launch_row_scale_copy(out, out, D.scale_ord, D.n, nrhs, st);
     return;

@@ -180,11 +180,12 @@ void launch_solve_small(const int4* info, const int64_t* ipx, const int* levptr,
 // the same sweeps for every system of a block-diagonal batch, one workgroup
 // per system (sysd: 6 ints per system, see solve_small.hip; its level
 // pointers index info / ipx); systems of at most fit_cols rows keep their
-// block in LDS, the others in xg (n x nrhs values of T in memory)
+// block in LDS, the others (up to max_cols rows) in xg (n x nrhs values of T
+// in memory)
 template <typename T>
 void launch_solve_batch(const int* sysd, int nsys, const int4* info, const int64_t* ipx, const int* levptr,
-                        const int* mode, int fit_cols, int maxlev, const SnArgs& a, const T* valL, const T* dval,
-                        const double* in, double* out, int nrhs, const double* active, int64_t astride, T* xg,
+                        const int* mode, int fit_cols, int max_cols, int maxlev, const SnArgs& a, const T* valL,
+                        const T* dval, const double* in, double* out, int nrhs, const double* active, int64_t astride, T* xg,
                         hipStream_t st);
 // per-column dot products out[c] = sum_i a(i, c) b(i, c) (rows interleaved by
 // column), reduced in a fixed order through at most nblk partials

@@ -372,12 +372,20 @@ __device__ void ss_forward_wg(const int4 I, int64_t px, const SnArgs& a, const T
       for (int c = 0; c < NR; ++c) acc[c] = (T)0;
       int j = ja;
       if (blk == blk0) {
+        if (ja + PF <= jb) {  // without a branch per column the reads of x go out together
 #pragma unroll
-        for (int u = 0; u < PF; ++u)
-          if (ja + u < jb) {
+          for (int u = 0; u < PF; ++u) {
 #pragma unroll
             for (int c = 0; c < NR; ++c) acc[c] += pf[u] * x.ld((c0 + cb + ja + u) * NR + c);
           }
+        } else {
+#pragma unroll
+          for (int u = 0; u < PF; ++u)
+            if (ja + u < jb) {
+#pragma unroll
+              for (int c = 0; c < NR; ++c) acc[c] += pf[u] * x.ld((c0 + cb + ja + u) * NR + c);
+            }
+        }
         j = min(jb, ja + PF);
       }
       if (ok) {
@@ -453,11 +461,19 @@ __device__ void ss_backward_wg(const int4 I, int64_t px, const SnArgs& a, const 
           lab[u] = q < qe ? (q < w ? c0 + (int)q : a.rows[pis + q]) : 0;
           l[u] = q < qe ? col[q] : (T)0;
         }
+        if (q0 + UF <= qe) {
 #pragma unroll
-        for (int u = 0; u < UF; ++u) {
-          if (q0 + u < qe) {
+          for (int u = 0; u < UF; ++u) {
 #pragma unroll
             for (int c = 0; c < NR; ++c) acc[c] += l[u] * x.ld(lab[u] * NR + c);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < UF; ++u) {
+            if (q0 + u < qe) {
+#pragma unroll
+              for (int c = 0; c < NR; ++c) acc[c] += l[u] * x.ld(lab[u] * NR + c);
+            }
           }
         }
       }
@@ -499,8 +515,12 @@ __device__ void ss_backward_wg(const int4 I, int64_t px, const SnArgs& a, const 
 // copies; each wave loads the description of its first supernode of the
 // next level before working on the current one, so a level costs one
 // dependent round of value loads instead of four.
+// Inlined into each kernel by force: as a function, called from two, it kept
+// 230 to 450 bytes a lane in scratch.  The sweep with the block in memory
+// (KKT of a 10^3 grid, 1 / 4 / 8 right-hand sides): FP64 236 / 476 / 1000 ->
+// 198 / 332 / 869 us, FP32 191 / 305 / 870 -> 178 / 269 / 531.
 template <typename T, int NR, bool XG>
-__device__ inline void ss_sweeps(const int4* info, const int64_t* ipx, const int* lp, const int* lm, int nlev,
+__device__ __forceinline__ void ss_sweeps(const int4* info, const int64_t* ipx, const int* lp, const int* lm, int nlev,
                                  int col0, int ncol, const SnArgs& a, const T* valL, const T* dval, const double* in,
                                  double* out, const XBlock<T, XG>& x, T* tile, T* red) {
   const int n = a.n, t = threadIdx.x, wv = t >> 6, ln = t & 63;
@@ -644,8 +664,9 @@ __global__ __launch_bounds__(SS_THREADS) void k_solve_small(const int4* info, co
 // sysd[6g ..] = (first level pointer, first mode, levels, first column,
 // columns, -); its level pointers index info / ipx directly.  A system whose
 // block has at most fit_elems values is kept in LDS, a larger one in xg (the
-// same rows of an n x NR block in memory).
-template <typename T, int NR>
+// same rows of an n x NR block in memory).  MEM = false, every system fits:
+// without the second form beside it the first one's code is up to 3% faster.
+template <typename T, int NR, bool MEM>
 __global__ __launch_bounds__(SS_THREADS) void k_solve_batch(const int* sysd, const int4* info, const int64_t* ipx,
                                                             const int* levptr, const int* mode, int fit_elems,
                                                             int maxlev, SnArgs a, const T* valL, const T* dval,
@@ -668,10 +689,10 @@ __global__ __launch_bounds__(SS_THREADS) void k_solve_batch(const int* sysd, con
   int* lm = lp + maxlev + 1;
   for (int i = t; i <= nlev; i += SS_THREADS) lp[i] = levptr[lpo + i];
   for (int i = t; i < nlev; i += SS_THREADS) lm[i] = mode[mdo + i];
-  if ((int64_t)ncol * NR <= fit_elems) {
+  if (!MEM || (int64_t)ncol * NR <= fit_elems) {
     const XBlock<T, false> x{lds, (int64_t)col0 * NR};
     ss_sweeps<T, NR, false>(info, ipx, lp, lm, nlev, col0, ncol, a, valL, dval, in, out, x, tile, red);
-  } else {
+  } else if constexpr (MEM) {
     const XBlock<T, true> x{xg, 0};
     ss_sweeps<T, NR, true>(info, ipx, lp, lm, nlev, col0, ncol, a, valL, dval, in, out, x, tile, red);
   }
@@ -706,20 +727,20 @@ void solve_small_nr(const int4* info, const int64_t* ipx, const int* levptr, con
   HIP_LAUNCH_CHECK("solve_small");
 }
 
-template <typename T, int NR>
+template <typename T, int NR, bool MEM>
 void solve_batch_nr(const int* sysd, int nsys, const int4* info, const int64_t* ipx, const int* levptr,
                     const int* mode, int fit_elems, int maxlev, const SnArgs& a, const T* valL, const T* dval,
                     const double* in, double* out, const double* active, int64_t astride, T* xg, hipStream_t st) {
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute((const void*)k_solve_batch<T, NR>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)k_solve_batch<T, NR, MEM>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)(SOLVE_SMALL_LDS + ss_lds<T>(0, MAX_RHS, SOLVE_SMALL_LEVELS))) != hipSuccess)
       throw std::runtime_error("solve_batch: LDS attribute");
     attr = true;
   }
   const size_t lds = sizeof(T) * (((size_t)fit_elems + 1) & ~(size_t)1) + ss_lds<T>(0, NR, maxlev);
-  k_solve_batch<T, NR><<<nsys, SS_THREADS, lds, st>>>(sysd, info, ipx, levptr, mode, fit_elems, maxlev, a, valL,
-                                                      dval, in, out, active, astride, xg);
+  k_solve_batch<T, NR, MEM><<<nsys, SS_THREADS, lds, st>>>(sysd, info, ipx, levptr, mode, fit_elems, maxlev, a, valL,
+                                                           dval, in, out, active, astride, xg);
   HIP_LAUNCH_CHECK("solve_batch");
 }
 
@@ -727,16 +748,20 @@ void solve_batch_nr(const int* sysd, int nsys, const int4* info, const int64_t* 
 
 template <typename T>
 void launch_solve_batch(const int* sysd, int nsys, const int4* info, const int64_t* ipx, const int* levptr,
-                        const int* mode, int fit_cols, int maxlev, const SnArgs& a, const T* valL, const T* dval,
-                        const double* in, double* out, int nrhs, const double* active, int64_t astride, T* xg,
+                        const int* mode, int fit_cols, int max_cols, int maxlev, const SnArgs& a, const T* valL,
+                        const T* dval, const double* in, double* out, int nrhs, const double* active, int64_t astride, T* xg,
                         hipStream_t st) {
   const int64_t fit = (int64_t)fit_cols * nrhs;
   if (nsys < 1 || nrhs < 1 || nrhs > MAX_RHS || maxlev < 1 || maxlev > SOLVE_SMALL_LEVELS ||
       sizeof(T) * (size_t)fit > SOLVE_SMALL_LDS || !xg)
     throw std::invalid_argument("solve_batch: schedule or block does not fit the workgroup's LDS");
   const int fe = (int)fit;
-#define SB(NR) solve_batch_nr<T, NR>(sysd, nsys, info, ipx, levptr, mode, fe, maxlev, a, valL, dval, in, out, active, \
-                                     astride, xg, st)
+#define SB(NR)                                                                                                       \
+  max_cols <= fit_cols                                                                                                \
+      ? solve_batch_nr<T, NR, false>(sysd, nsys, info, ipx, levptr, mode, fe, maxlev, a, valL, dval, in, out, active, \
+                                     astride, xg, st)                                                                 \
+      : solve_batch_nr<T, NR, true>(sysd, nsys, info, ipx, levptr, mode, fe, maxlev, a, valL, dval, in, out, active,  \
+                                    astride, xg, st)
   switch (nrhs) {
     case 1: SB(1); break;
     case 2: SB(2); break;
@@ -770,10 +795,10 @@ void launch_solve_small(const int4* info, const int64_t* ipx, const int* levptr,
 }
 
 template void launch_solve_batch<double>(const int*, int, const int4*, const int64_t*, const int*, const int*, int,
-                                         int, const SnArgs&, const double*, const double*, const double*, double*, int,
+                                         int, int, const SnArgs&, const double*, const double*, const double*, double*, int,
                                          const double*, int64_t, double*, hipStream_t);
 template void launch_solve_batch<float>(const int*, int, const int4*, const int64_t*, const int*, const int*, int, int,
-                                        const SnArgs&, const float*, const float*, const double*, double*, int,
+                                        int, const SnArgs&, const float*, const float*, const double*, double*, int,
                                         const double*, int64_t, float*, hipStream_t);
 template void launch_solve_small<double>(const int4*, const int64_t*, const int*, const int*, int, const SnArgs&,
                                          const double*, const double*, const double*, double*, int, const double*,
