@@ -25,6 +25,7 @@
 namespace lblg {
 
 typedef short s4 __attribute__((ext_vector_type(4)));
+typedef short s8 __attribute__((ext_vector_type(8)));
 
 __device__ inline unsigned short f2bf(float f) {  // round to nearest even
   unsigned u = __float_as_uint(f);
@@ -137,12 +138,12 @@ static void gemm(int M, int N, int K, const TA* A, int64_t sa0, int64_t sa1, con
 // A minibatch has few rows: 64 x 64 tiles give 16 workgroups on 256 CUs and a
 // chain of K / 32 staged chunks, 64 to 73 us at 64 x 1024 x 1024.  The chain
 // of MFMAs itself is short (K / 16 of them), the loads are what it waits for,
-// so one wave takes one 16 x 16 tile, reads its operands lane by lane without
-// LDS and has WU to 2 WU slices in flight: 10.8 us with k contiguous in W,
-// 20.1 us with j contiguous.  Eight or sixteen slices, or four waves a
-// workgroup, were no faster there (10.5 to 18 us).
+// so one wave takes one 16 x 16 tile, reads its operands lane by lane and has
+// the next slices in flight: 9.0 us with k contiguous in W, 11.4 us with j
+// contiguous (13 and 17 us with operands that are not in the L2).  With k
+// contiguous 4 or 16 slices take 9.7 and 8.8 us (15 and 12), 16 lose where K
+// is short (4.2 against 3.3 us at K = 32); four waves a workgroup took 18 us.
 // --------------------------------------------------------------------------
-constexpr int WU = 4;  // slices loaded together
 // four consecutive k of A's row, zero beyond K
 template <bool VEC>
 __device__ inline f4 load_a(const float* row, int k, int K) {
@@ -152,29 +153,49 @@ __device__ inline f4 load_a(const float* row, int k, int K) {
   for (int e = 0; e < 4; ++e) v[e] = k + e < K ? row[k + e] : 0.f;
   return v;
 }
+// four consecutive k of W's column (VEC: contiguous, K a multiple of four)
 template <bool VEC>
 __device__ inline s4 load_w(const unsigned short* col, int64_t sw0, int k, int K) {
-  if (VEC && sw0 == 1) return k < K ? *reinterpret_cast<const s4*>(col + k) : s4{0, 0, 0, 0};
+  if (VEC) return k < K ? *reinterpret_cast<const s4*>(col + k) : s4{0, 0, 0, 0};
   s4 r;
   for (int e = 0; e < 4; ++e) r[e] = k + e < K ? (short)col[(int64_t)(k + e) * sw0] : (short)0;
   return r;
 }
-template <bool VEC>
+// How W is read: element by element; along k, four at a time; or along j
+// (sw0 a multiple of 8), where a lane takes 16 columns of one k and the wave
+// turns them in LDS: two wide loads a lane for four slices in place of sixteen
+// two-byte ones, 20 -> 11.4 us.
+enum { W_ELEM = 0, W_ALONG_K = 1, W_ALONG_J = 2 };
+// slices loaded together
+constexpr int weight_slices(int wr) { return wr == W_ALONG_K ? 8 : 4; }
+constexpr int WTP = 24;  // LDS row of one k: 16 columns, the four k-groups of a read in different banks
+template <bool VEC, int WR>
 __global__ __launch_bounds__(64) void k_gemm_weight(int M, int N, int K, const float* A, int lda,
                                                     const unsigned short* W, int64_t sw0, int64_t sw1, float* C,
                                                     int ldc, Epilogue f) {
+  constexpr int WU = weight_slices(WR);
+  __shared__ __align__(16) unsigned short tile[WR == W_ALONG_J ? 16 * WU * WTP : 1];
+  static_assert(WR != W_ALONG_J || 16 * WU == 64, "a lane of the wave per k of a round");
   const int ln = threadIdx.x, li = ln & 15, lk = 4 * (ln >> 4);
   const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16;
   // rows and columns beyond the matrix read the last one and are not stored
   const float* ar = A + (int64_t)min(i0 + li, M - 1) * lda;
   const unsigned short* wc = W + (int64_t)min(j0 + li, N - 1) * sw1;
+  const bool turn = WR == W_ALONG_J && j0 + 16 <= N;  // the last columns' tile: element by element
   f4 acc = {0.f, 0.f, 0.f, 0.f}, a[WU];
   s4 b[WU];
+  s8 w0, w1;
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < WU; ++u) {
-      a[u] = load_a<VEC>(ar, k0 + 16 * u + lk, K);
-      b[u] = load_w<VEC>(wc, sw0, k0 + 16 * u + lk, K);
+    for (int u = 0; u < WU; ++u) a[u] = load_a<VEC>(ar, k0 + 16 * u + lk, K);
+    if (turn) {
+      const s8* row = reinterpret_cast<const s8*>(W + (int64_t)min(k0 + ln, K - 1) * sw0 + j0);
+      w0 = row[0];
+      w1 = row[1];
+      if (k0 + ln >= K) w0 = w1 = s8{0, 0, 0, 0, 0, 0, 0, 0};
+    } else {
+#pragma unroll
+      for (int u = 0; u < WU; ++u) b[u] = load_w<WR == W_ALONG_K>(wc, sw0, k0 + 16 * u + lk, K);
     }
   };
   fetch(0);
@@ -182,9 +203,19 @@ __global__ __launch_bounds__(64) void k_gemm_weight(int M, int N, int K, const f
     f4 x[WU];
     s4 y[WU];
 #pragma unroll
-    for (int u = 0; u < WU; ++u) {
-      x[u] = a[u];
-      y[u] = b[u];
+    for (int u = 0; u < WU; ++u) x[u] = a[u];
+    if (turn) {
+      __syncthreads();  // one wave: orders its reads of the round before against these stores
+      *reinterpret_cast<s8*>(tile + ln * WTP) = w0;
+      *reinterpret_cast<s8*>(tile + ln * WTP + 8) = w1;
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < WU; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[u][e] = (short)tile[(16 * u + lk + e) * WTP + li];
+    } else {
+#pragma unroll
+      for (int u = 0; u < WU; ++u) y[u] = b[u];
     }
     fetch(k0 + 16 * WU);  // the next slices' loads beside these slices' MFMAs (zeros beyond K)
 #pragma unroll
@@ -204,22 +235,24 @@ static void gemm_weight(int M, int N, int K, const float* A, const unsigned shor
                         float* C, const Epilogue& f, hipStream_t st) {
   // Many rows fill the chip with 64 x 64 tiles too, which read each operand a
   // quarter as often.  64 x 64 tiles / one wave a tile, us, K = 1024, N = 1024:
-  // k contiguous in W, M = 64: 73 / 10.8, 1024: 80 / 60, 2048: 132 / 116,
-  // 4096: 233 / 226; j contiguous (two-byte loads), M = 64: 64 / 20,
-  // 1024: 100 / 45, 2048: 101 / 87, 4096: 155 / 168; 1024 x 4000: 154 / 172.
+  // k contiguous in W, M = 64: 73 / 9.0, 1024: 80 / 60, 2048: 131 / 115,
+  // 4096: 232 / 225; j contiguous, M = 64: 64 / 11.4, 1024: 99 / 50,
+  // 2048: 100 / 95, 4096: 155 / 181; 1024 x 4000: 155 / 188.
   // (The 16-row tiles also end at the grid's 65,535 rows of workgroups.)
   if ((sw0 != 1 && (int64_t)M * N > (int64_t)1 << 21) || M > 65535 * 16) {
     gemm(M, N, K, A, K, 1, W, sw0, sw1, C, N, st, f);
     return;
   }
   const dim3 grid((N + 15) / 16, (M + 15) / 16);
-  // four-element loads: rows of A (and of W, read along k) on their alignment
-  const bool vec = K % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
-                   (sw0 != 1 || (sw1 % 4 == 0 && reinterpret_cast<uintptr_t>(W) % 8 == 0));
-  if (vec)
-    k_gemm_weight<true><<<grid, 64, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, f);
+  // wide loads: rows of A and of W on their alignment
+  const bool va = K % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0;
+  const bool wk = sw0 == 1 && K % 4 == 0 && sw1 % 4 == 0 && reinterpret_cast<uintptr_t>(W) % 8 == 0;
+  const bool wj = sw1 == 1 && sw0 % 8 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0;
+  auto go = [&](auto kernel) { kernel<<<grid, 64, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, f); };
+  if (va)
+    go(wk ? k_gemm_weight<true, W_ALONG_K> : wj ? k_gemm_weight<true, W_ALONG_J> : k_gemm_weight<true, W_ELEM>);
   else
-    k_gemm_weight<false><<<grid, 64, 0, st>>>(M, N, K, A, K, W, sw0, sw1, C, N, f);
+    go(wj ? k_gemm_weight<false, W_ALONG_J> : k_gemm_weight<false, W_ELEM>);
   HIP_LAUNCH_CHECK("gemm_weight");
 }
 

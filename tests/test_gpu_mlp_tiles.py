@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dims,batch", [((4, 36, 64, 1), 1), ((32, 33, 31, 65), 33), ((8, 100, 60, 33), 64),
-                                        ((17, 130, 260, 96), 31)])
+                                        ((17, 130, 260, 96), 31), ((16, 136, 264, 96), 40),
+                                        ((16, 136, 264, 97), 33)])  # 264: wide reads across, a last tile of 8
 def test_gradients_and_predictions(dims, batch):
     print(f"case mlp tiles dims={dims} batch={batch}", flush=True)
     net, p = make_net(dims, batch, seed=sum(dims))
