@@ -372,20 +372,12 @@ __device__ void ss_forward_wg(const int4 I, int64_t px, const SnArgs& a, const T
       for (int c = 0; c < NR; ++c) acc[c] = (T)0;
       int j = ja;
       if (blk == blk0) {
-        if (ja + PF <= jb) {  // without a branch per column the reads of x go out together
 #pragma unroll
-          for (int u = 0; u < PF; ++u) {
+        for (int u = 0; u < PF; ++u)
+          if (ja + u < jb) {
 #pragma unroll
             for (int c = 0; c < NR; ++c) acc[c] += pf[u] * x.ld((c0 + cb + ja + u) * NR + c);
           }
-        } else {
-#pragma unroll
-          for (int u = 0; u < PF; ++u)
-            if (ja + u < jb) {
-#pragma unroll
-              for (int c = 0; c < NR; ++c) acc[c] += pf[u] * x.ld((c0 + cb + ja + u) * NR + c);
-            }
-        }
         j = min(jb, ja + PF);
       }
       if (ok) {
@@ -461,19 +453,11 @@ __device__ void ss_backward_wg(const int4 I, int64_t px, const SnArgs& a, const 
           lab[u] = q < qe ? (q < w ? c0 + (int)q : a.rows[pis + q]) : 0;
           l[u] = q < qe ? col[q] : (T)0;
         }
-        if (q0 + UF <= qe) {
 #pragma unroll
-          for (int u = 0; u < UF; ++u) {
+        for (int u = 0; u < UF; ++u) {
+          if (q0 + u < qe) {
 #pragma unroll
             for (int c = 0; c < NR; ++c) acc[c] += l[u] * x.ld(lab[u] * NR + c);
-          }
-        } else {
-#pragma unroll
-          for (int u = 0; u < UF; ++u) {
-            if (q0 + u < qe) {
-#pragma unroll
-              for (int c = 0; c < NR; ++c) acc[c] += l[u] * x.ld(lab[u] * NR + c);
-            }
           }
         }
       }
@@ -517,12 +501,12 @@ __device__ void ss_backward_wg(const int4 I, int64_t px, const SnArgs& a, const 
 // dependent round of value loads instead of four.
 // Inlined into each kernel by force: as a function, called from two, it kept
 // 230 to 450 bytes a lane in scratch.  The sweep with the block in memory
-// (KKT of a 10^3 grid, 1 / 4 / 8 right-hand sides): FP64 236 / 476 / 1000 ->
-// 198 / 332 / 869 us, FP32 191 / 305 / 870 -> 178 / 269 / 531.
+// (KKT of a 10^3 grid, 1 / 4 / 8 right-hand sides): FP64 243 / 473 / 994 ->
+// 193 / 334 / 861 us, FP32 169 / 305 / 821 -> 155 / 272 / 550.
 template <typename T, int NR, bool XG>
-__device__ __forceinline__ void ss_sweeps(const int4* info, const int64_t* ipx, const int* lp, const int* lm, int nlev,
-                                 int col0, int ncol, const SnArgs& a, const T* valL, const T* dval, const double* in,
-                                 double* out, const XBlock<T, XG>& x, T* tile, T* red) {
+__device__ __forceinline__ void ss_sweeps(const int4* info, const int64_t* ipx, const int* lp, const int* lm,
+                                          int nlev, int col0, int ncol, const SnArgs& a, const T* valL, const T* dval,
+                                          const double* in, double* out, const XBlock<T, XG>& x, T* tile, T* red) {
   const int n = a.n, t = threadIdx.x, wv = t >> 6, ln = t & 63;
   const int64_t e0 = (int64_t)col0 * NR, e1 = (int64_t)(col0 + ncol) * NR;
   for (int64_t i = e0 + t; i < e1; i += SS_THREADS) x.st(i, (T)in[i]);
@@ -749,8 +733,8 @@ void solve_batch_nr(const int* sysd, int nsys, const int4* info, const int64_t* 
 template <typename T>
 void launch_solve_batch(const int* sysd, int nsys, const int4* info, const int64_t* ipx, const int* levptr,
                         const int* mode, int fit_cols, int max_cols, int maxlev, const SnArgs& a, const T* valL,
-                        const T* dval, const double* in, double* out, int nrhs, const double* active, int64_t astride, T* xg,
-                        hipStream_t st) {
+                        const T* dval, const double* in, double* out, int nrhs, const double* active, int64_t astride,
+                        T* xg, hipStream_t st) {
   const int64_t fit = (int64_t)fit_cols * nrhs;
   if (nsys < 1 || nrhs < 1 || nrhs > MAX_RHS || maxlev < 1 || maxlev > SOLVE_SMALL_LEVELS ||
       sizeof(T) * (size_t)fit > SOLVE_SMALL_LDS || !xg)
