@@ -329,12 +329,17 @@ __global__ __launch_bounds__(NT, (panel_waves<T, NT, NBM, ONE>())) void k_bk_wid
   // a(i,j) -= sum_c L(i,c) W(j,c); inside the sub-block every wave computes
   // the diagonal rows itself, so the steps need no block barrier.
   // What bounds the panel is the chain of nbe dependent steps, so a step
-  // keeps its operands in registers.  Per 64-column FP64 panel of the 64^3
-  // KKT (476 panels, workgroup 0, phase stamps): load 8.6 us, MFMA 10.8,
-  // steps 16.4 (0.26 us each), exchange 2.6, pivot search 6.9 (averaged; 6
-  // panels take it), write 9.8.  With the columns in LDS and one sum per
-  // step over the sub-block's earlier columns a launch took 115 us, now 58
-  // (FP32 panels of the 48^3 KKT: 129 -> 59).
+  // keeps its operands in registers.  Per 64-column FP64 panel of a 64^3 KKT
+  // (476 panels, workgroup 0, phase stamps): load 8.1 us, MFMA 11.4, steps
+  // 23.3 (0.36 us each), exchange 1.8, pivot search 3.6 (averaged; 6 panels
+  // take it), restore and interchanges 1.5, write 9.1.  With the columns in
+  // LDS and one sum per step over the sub-block's earlier columns a launch
+  // took 115 us on average, now 60 (kernel traces; FP32 panels of a 48^3 KKT:
+  // 124 -> 63; where 14 of 476 panels take the search, FP64 68).
+  // The price is registers: 252 vector registers for the cooperative FP64
+  // form (106 before) and 150 to 290 scalar ones kept in vector lanes, which
+  // costs no residency (the LDS allows one workgroup a CU); the 1024-thread
+  // form has 128 and spills 19 of them in FP64 (3 in FP32).
   //
   // ---- Pivot step.  One step of the search at column kr on left-looking
   // sums over the eliminated columns: a record exchange per step, a second
@@ -1142,9 +1147,11 @@ template void launch_bk_wide<double>(const WideSn&, int, int, int, int, int, int
 template void launch_bk_wide<float>(const WideSn&, int, int, int, int, int, int, float*, float*, int*, float*,
                                     int*, int*, int*, int*, uint64_t*, uint32_t, int*, hipStream_t);
 
-// One-workgroup panels.  What bounds them is the chain of column steps, 0.26
-// to 0.3 us each where every pivot is accepted in place and about 2.4 us per
-// column where every column needs the search.  Measured per launch, before
+// One-workgroup panels.  What bounds them is the chain of column steps, about
+// 0.36 us each where every pivot is accepted in place; a block that searches
+// at every column takes 3.4 to 4.7 us a column, launches and trailing updates
+// included (65 to 256 columns), 0.94 to 1.3 times the speed of the panels
+// before, by the width.  Measured per launch, before
 // (columns summed left-looking from LDS or memory, 31 per launch) and now:
 // 33^3 KKT 83-138 us -> 43 (64 columns) / 30 (32) / 23 (16), 24 x 150
 // block-indefinite 82-102 us -> 234 / 139 / 98, that is 11.1 -> 9.1 ms a
