@@ -175,7 +175,7 @@ __global__ __launch_bounds__(64) void k_gemm_weight(int M, int N, int K, const f
                                                     int ldc, Epilogue f) {
   constexpr int WU = weight_slices(WR);
   __shared__ __align__(16) unsigned short tile[WR == W_ALONG_J ? 16 * WU * WTP : 1];
-  static_assert(WR != W_ALONG_J || 16 * WU == 64, "a lane of the wave per k of a round");
+  static_assert(WR != W_ALONG_J || 16 * WU == 64, "a lane of the wave per k");
   const int ln = threadIdx.x, li = ln & 15, lk = 4 * (ln >> 4);
   const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16;
   // rows and columns beyond the matrix read the last one and are not stored
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(64) void k_gemm_weight(int M, int N, int K, const f
 #pragma unroll
     for (int u = 0; u < WU; ++u) x[u] = a[u];
     if (turn) {
-      __syncthreads();  // one wave: orders its reads of the round before against these stores
+      __syncthreads();  // one wave: orders its reads of the slices before against these stores
       *reinterpret_cast<s8*>(tile + ln * WTP) = w0;
       *reinterpret_cast<s8*>(tile + ln * WTP + 8) = w1;
       __syncthreads();
